@@ -241,7 +241,8 @@ static int make_gtype(rbc3d_ctx *c, int nlat, GridType **out) {
   RBC_TRY(upload(g->d_thG, thG, st));
   RBC_TRY(upload(g->d_phiG, phiG, st));
   RBC_TRY(upload(g->d_pwt, wL, st));
-  // same-surface mask MaskFunc(DistOnSphere/radius) by (ilat_i, ilat_j, ilon_j - ilon_i)
+  // same-surface mask MaskFunc(DistOnSphere/radius) by (ilat_i, ilon_j - ilon_i, ilat_j):
+  // a row is the order of a cell's nodes, shifted to the target's longitude
   std::vector<double> mk((size_t)nl * nl * nn);
   for (int a = 0; a < nl; a++)
     for (int b = 0; b < nl; b++)
@@ -249,7 +250,7 @@ static int make_gtype(rbc3d_ctx *c, int nlat, GridType **out) {
         double th0 = g->th[a], th1 = g->th[b], phi0 = g->phi[0], phi1 = g->phi[d];
         double dd = cos(th0 - th1) - sin(th0) * sin(th1) * (1. - cos(phi0 - phi1));
         dd = std::min(1., std::max(-1., dd));
-        mk[((size_t)a * nl + b) * nn + d] = mask_tab(mt, acos(dd) / g->radius);
+        mk[((size_t)a * nn + d) * nl + b] = mask_tab(mt, acos(dd) / g->radius);
       }
   RBC_TRY(upload(g->d_mask, mk, st));
   std::vector<float> mkf(mk.begin(), mk.end());  // the split form's pair kernel
@@ -439,6 +440,8 @@ extern "C" int rbc3d_create(const rbc3d_conf *conf, rbc3d_ctx **out) {
     mt[i] = mask_exact((double)i / RBC_NTAB);
   }
   c->r_eps = 1.e-3 * sqrt(alpha / RBC_PI);
+  // one more entry, so that kernels may read the pair (i, i + 1) up to i = RBC_NTAB
+  for (auto *t : {&t1, &t2, &t3}) t->push_back(0.);
   int r = upload(c->d_sl1, t1, c->stream);
   if (!r) r = upload(c->d_sl2, t2, c->stream);
   if (!r) r = upload(c->d_dl1, t3, c->stream);
@@ -562,7 +565,7 @@ extern "C" int rbc3d_destroy(rbc3d_ctx *c) {
     b->release();
   for (DBuf<int> *b : {&c->d_node_cell, &c->d_node_ll, &c->d_src_bin, &c->d_src_order,
                        &c->d_bin_start, &c->d_tmp_i, &c->d_tindx, &c->d_tact, &c->d_tbin,
-                       &c->d_torder, &c->d_tbin_start, &c->d_chunk_off, &c->d_nbr_cnt,
+                       &c->d_torder, &c->d_tbin_start, &c->d_chunk_off, &c->d_clus, &c->d_nbr_cnt,
                        &c->d_nbr_cell, &c->d_nbr_node, &c->d_cell_cand, &c->d_work, &c->d_work_cnt, &c->d_flag,
                        &c->d_cellbin_start, &c->d_cellbin_order, &c->d_pme_key, &c->d_pme_order,
                        &c->d_pme_start, &c->wall.d_e2v, &c->wall.d_glb, &c->wall.d_bin_start,

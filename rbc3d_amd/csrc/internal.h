@@ -85,7 +85,7 @@ struct GridType {
   DBuf<double> d_Dm;     // periodic derivative matrix, length 2 nlat, [p][q]
   DBuf<double> d_Dn;     // periodic derivative matrix, length nlon, [p][q]
   DBuf<double> d_thG, d_phiG, d_pwt;  // polar patch: [node][irad + nrad*iazm], weights
-  DBuf<double> d_mask;   // same-surface mask [ilat_i][ilat_j][dlon]
+  DBuf<double> d_mask;   // same-surface mask [ilat_i][dlon][ilat_j]
   DBuf<float> d_maskf;   // the same in FP32
   DBuf<double> d_proj;   // projection tables (RBC_PJ_*)
   // split form: the Legendre tables as three BF16 terms, [3][mmax][nlat][nlat] each
@@ -227,6 +227,7 @@ struct rbc3d_ctx {
   // target scratch
   DBuf<double> d_tx, d_tA, d_v, d_vacc;
   DBuf<int> d_tindx, d_tact, d_tbin, d_torder, d_tbin_start, d_chunk_off;
+  DBuf<int> d_clus;  // the pair kernel's target clusters: (fine bin, first sorted target)
   DBuf<int> d_nbr_cnt, d_nbr_cell, d_nbr_node;
   DBuf<int> d_cell_cand;  // per cell: candidate neighbouring cells, then their counts
   DBuf<double> d_nbr_dist;
@@ -262,6 +263,8 @@ struct rbc3d_ctx {
   WallData wall;
   // per-grid-type table pointers for the kernels
   DBuf<const double *> d_tp_ptr;
+  DBuf<double> d_maskcat;  // 1 - every grid type's d_mask, back to back
+  DBuf<int> d_maskoff;     // where each starts
   DBuf<const float *> d_tp_maskf;  // FP32 mask table per grid type
   DBuf<int> d_tp_int;
   size_t tp_ntypes = 0;

@@ -8,15 +8,15 @@
 //   the periodic linear double-layer term (AddLinearInt, common/ModIntOnRbcs.F90:162-201).
 //
 // Layout: sources are sorted by cell-list bin (stable, so ascending index inside a
-// bin); targets are binned the same way.  The pair kernel gives one workgroup to a
-// chunk of up to 256 targets of one bin and streams the sources of the 27
-// neighbouring bins through LDS tiles.  Each lane owns one target, accumulates in
-// registers and writes once: no atomics, a fixed summation order per target.
+// bin); targets are binned the same way, in Z order inside a bin.  The pair kernels
+// stream the sources of the neighbouring bins through LDS past a few targets of one bin,
+// accumulate in registers and write once: no atomics, a fixed summation order per target.
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 #include "internal.h"
 #include "surf_core.h"
@@ -134,14 +134,17 @@ int rbc_hash_sort(rbc3d_ctx *c, int n, const double *d_x, int ldx, int *d_bin, i
 }
 
 // the pair kernel's grid (fine bins)
-static int fine_sort(rbc3d_ctx *c, int n, const double *d_x, int ldx, int *d_bin, int *d_order,
-                     int *d_bin_start) {
+static HashGeom fine_geom(const rbc3d_ctx *c) {
   HashGeom hg;
   for (int d = 0; d < 3; d++) {
     hg.Nc[d] = c->Nf[d];
     hg.iLbNc[d] = c->iLbNf[d];
   }
-  return hash_sort_grid(c, hg, c->nfbins, n, d_x, ldx, d_bin, d_order, d_bin_start);
+  return hg;
+}
+static int fine_sort(rbc3d_ctx *c, int n, const double *d_x, int ldx, int *d_bin, int *d_order,
+                     int *d_bin_start) {
+  return hash_sort_grid(c, fine_geom(c), c->nfbins, n, d_x, ldx, d_bin, d_order, d_bin_start);
 }
 
 // hoc/next from the sorted list, with the ghost layers of HashTable_Build
@@ -332,26 +335,34 @@ extern "C" int rbc3d_hashtable_build_noalloc(const int Nc[3], const double iLbNc
 // ---------------------------------------------------------------------------
 // source list on cells
 
-// sorted source records, SoA with stride np: x,y,z, f(3), g(3), a3(3), Bcoef  (13)
+// sorted source records: x, y, z with stride np, then per source (f, 0), then per source
+// (g Bcoef, a3); np is even, so the last two are 16-byte aligned
 #define SREC 13
+#define SREC_F(np) (3 * (size_t)(np))
+#define SREC_G(np) (7 * (size_t)(np))
+// set in a record's node when the source lies outside the box [0, Lb)
+#define SRC_OUT (1u << 31)
 
 __global__ void k_src_records(int np, const int *__restrict__ order, const double *__restrict__ x,
                               const double *__restrict__ fs, const double *__restrict__ gs,
                               const double *__restrict__ a3, const CellRec *__restrict__ cells,
                               const int *__restrict__ node_cell, const int *__restrict__ node_ll,
-                              double *__restrict__ rec, int *__restrict__ rec_meta) {
+                              HashGeom fine, double *__restrict__ rec, int *__restrict__ rec_meta) {
   int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= np) return;
   int p = order[k];
+  const double B = cells[node_cell[p]].Bcoef;
+  bool out = false;
   for (int d = 0; d < 3; d++) {
-    rec[k + (size_t)np * d] = x[p + (size_t)np * d];
-    rec[k + (size_t)np * (3 + d)] = fs[p + (size_t)np * d];
-    rec[k + (size_t)np * (6 + d)] = gs[p + (size_t)np * d];
-    rec[k + (size_t)np * (9 + d)] = a3[p + (size_t)np * d];
+    const double xd = x[p + (size_t)np * d], fl = floor(xd * fine.iLbNc[d]);  // as k_bins
+    out = out || fl < 0 || fl >= fine.Nc[d];
+    rec[k + (size_t)np * d] = xd;
+    rec[SREC_F(np) + 4 * (size_t)k + d] = fs[p + (size_t)np * d];
+    rec[SREC_G(np) + 6 * (size_t)k + d] = gs[p + (size_t)np * d] * B;
+    rec[SREC_G(np) + 6 * (size_t)k + 3 + d] = a3[p + (size_t)np * d];
   }
-  rec[k + (size_t)np * 12] = cells[node_cell[p]].Bcoef;
-  // sorted-position metadata [3][np]: node, cell, (ilat | ilon << 16)
-  rec_meta[k] = p;
+  // sorted-position metadata [3][np]: node (and SRC_OUT), cell, (ilat | ilon << 16)
+  rec_meta[k] = (int)((unsigned)p | (out ? SRC_OUT : 0u));
   rec_meta[k + (size_t)np] = node_cell[p];
   rec_meta[k + 2 * (size_t)np] = node_ll[p];
 }
@@ -493,8 +504,8 @@ int rbc_update_density(rbc3d_ctx *c, int which) {
   RBC_TRY(c->d_work.ensure(3 * (size_t)np + 1));
   k_src_records<<<(np + 255) / 256, 256, 0, st>>>(np, c->d_src_order.p, c->d_x.p, c->d_fs.p,
                                                   c->d_gs.p, c->d_a3.p, c->d_cells.p,
-                                                  c->d_node_cell.p, c->d_node_ll.p, c->d_src_rec.p,
-                                                  c->d_work.p);
+                                                  c->d_node_cell.p, c->d_node_ll.p, fine_geom(c),
+                                                  c->d_src_rec.p, c->d_work.p);
   HIP_TRY(hipGetLastError());
   return RBC3D_OK;
 }
@@ -507,56 +518,90 @@ int rbc_update_density(rbc3d_ctx *c, int which) {
 // minimum-image pair with rr <= rc (its bins are at least rc wide, or there are
 // three of them and all are visited), so the pair set is {rr <= rc} and any
 // conservative enumeration reproduces it: here the source bins within +-R of the
-// target bin whose box distance does not exceed rc.  A workgroup is one wavefront
-// owning up to 64 targets of one fine bin; sources stream through LDS in tiles.
+// target bin whose box distance does not exceed rc.
 
-#define PT 64    // targets per workgroup, one per lane
-#define PW 4     // wavefronts per workgroup, each taking every PW-th source of a tile
-#define PS 256   // sources per LDS tile
+#define PT 64    // targets per workgroup of the chunk kernels, one per lane
+#define PW 4     // their wavefronts per workgroup, each taking every PW-th source of a tile
+#define PS 256   // sources per LDS tile of the single-layer kernel
+#define PC 8     // targets per cluster (one wavefront's work item)
+#define PQ (64 / PC)  // source slots per evaluation step
+#define PCAP (64 + PQ)  // staged sources per wavefront
 
 struct PairArgs {
-  double Lb[3], iLb[3], iLbNf[3];
+  double Lb[3], iLb[3], iLbNf[3], w[3];  // box, 1/box, 1/bin width, bin width
   int Nf[3];
   int img;  // 1: periodic images from the visited bins (every dimension has >= 2R+3 bins)
-  double rc, rc2hi, rc2lo, reps2, tabscale, c1, c2;
+  double rc, rc2, rc2hi, rc2lo, rc2w, reps2, tabscale, c1, c2;  // rc2w: half width of the shell
   int np, nT, nfbins, nrbc, nrows;
   const int *rows;       // x-rows of source bins: packed (alo, ahi, o2, o3)
   const double *rec;     // sources sorted by fine bin (SREC x np)
-  const int *src_node;   // sorted position -> node, then cell, then (ilat | ilon << 16)
+  const int *src_node;   // sorted position -> node (SRC_OUT), then cell, then (ilat | ilon << 16)
   const int *bin_start;  // sources per fine bin
-  const int *node_cell, *node_ll;
   const CellRec *cells;
   const double *sl1, *sl2, *dl1;
   const double *const *mask;  // per grid type same-surface mask tables
+  const double *maskcat;      // 1 - mask, back to back, type g from maskoff[g]
+  const int *maskoff;
   const double *tx, *tA;
   const int *tindx, *tact, *torder, *tbin_start, *chunk_off;
+  const int *clus_off;   // clusters before each fine bin (clus_off[0] is the base)
+  const int2 *clus;      // cluster -> (fine bin, first sorted target)
+  int *ticket;           // per XCD: clusters of its range handed out after the first ones
   double *vpair;
   unsigned long long *stat;  // [0] in-cutoff pairs, [1] pair-set checksum
 };
 
-__global__ void k_chunks(int nbins, const int *__restrict__ tbin_start, int *chunk_cnt) {
+// per fine bin: 64-target chunks in cnt[0..nbins], PC-target clusters in
+// cnt[nbins + 1 .. 2 nbins + 1] (both end with a zero, so one scan of the whole array
+// gives both lists' offsets)
+__global__ void k_chunks(int nbins, const int *__restrict__ tbin_start, int *cnt) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b > nbins) return;
-  chunk_cnt[b] = b < nbins ? (tbin_start[b + 1] - tbin_start[b] + PT - 1) / PT : 0;
+  const int n = b < nbins ? tbin_start[b + 1] - tbin_start[b] : 0;
+  cnt[b] = (n + PT - 1) / PT;
+  cnt[nbins + 1 + b] = (n + PC - 1) / PC;
+}
+__global__ void k_clusters(int nbins, const int *__restrict__ tbin_start,
+                           const int *__restrict__ off, int2 *clus) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= nbins) return;
+  const int o = off[b] - off[0], n = off[b + 1] - off[b], t0 = tbin_start[b];
+  for (int k = 0; k < n; k++) clus[o + k] = make_int2(b, t0 + PC * k);
 }
 
-// SL: single-layer term present (c1 != 0); DL: double-layer term present (c2 != 0).
-// The workgroup's four wavefronts hold the same 64 targets and split every source
-// tile between them; their partial sums are added in wavefront order at the end.
-// Periodic images: the reference takes the minimum image of every candidate,
-// d - NINT(d / Lb) Lb.  When every dimension has at least 2R+3 fine bins, the image of
-// an in-cutoff pair is fixed by the bin walk: the source bin's wrap count k_run, the
-// target's box index kt (targets may lie outside [0, Lb)) and the source's (zero for a
-// source inside the box) give d = fl(xs - xi) + fl((k_run + kt) Lb), the same two
-// roundings as the reference's fl(fl(xs - xi) - fl(NINT * Lb)) with NINT = -(k_run +
-// kt); a candidate whose image differs is farther than rc either way.  Tiles holding a
-// source outside the box take the reference's formula.  In the image path the loader
-// keeps only the sources whose image comes within rc (plus a margin) of the chunk's
-// bounding sphere, packed in their order: about 30% of the candidates of a dense
-// packing pair with some target of the chunk, and the rest would each cost every lane
-// a distance test.  The pair set is unchanged.  The tiles take 26 KB of LDS,
-// so six workgroups fit a compute unit; the register budget is set to match (six
-// wavefronts per SIMD with a few spills measured 10% faster than four without).
+// target sort key: the fine bin, then (sub = 64) the position inside it on a 4^3 Z-order
+// grid, so that consecutive targets of a bin are close together; sub = 1: the bin alone
+__global__ void k_target_keys(int n, const double *__restrict__ x, HashGeom hg, int sub, int *key,
+                              int *idx) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double xi[3] = {x[i], x[i + (size_t)n], x[i + 2 * (size_t)n]};
+  int b1, b2, b3, z = 0;
+  hash_index3(xi, hg.Nc, hg.iLbNc, b1, b2, b3);
+  for (int d = 0; d < 3; d++) {
+    const double f = xi[d] * hg.iLbNc[d];
+    const int q = min(3, (int)((f - floor(f)) * 4.));
+    z |= ((q & 1) << d) | ((q >> 1) << (3 + d));
+  }
+  key[i] = sub * ((b1 - 1) + hg.Nc[0] * ((b2 - 1) + hg.Nc[1] * (b3 - 1))) + (sub > 1 ? z : 0);
+  idx[i] = i;
+}
+// bin_start[b] = first sorted position with key >= sub b
+__global__ void k_target_bin_start(int n, const int *__restrict__ skey, int nbins, int sub,
+                                   int *bin_start) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b > nbins) return;
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (skey[mid] < (long long)sub * b)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  bin_start[b] = lo;
+}
+
 // a value every lane of the wavefront holds, moved to scalar registers
 __device__ __forceinline__ double wave_uniform(double v) {
   const unsigned long long u = (unsigned long long)__double_as_longlong(v);
@@ -564,17 +609,505 @@ __device__ __forceinline__ double wave_uniform(double v) {
   const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
+// 1/sqrt(x), x > 0 normal, from the hardware estimate and one third-order step: with
+// e = 1 - x y^2, y (1 + e/2 + 3 e^2/8) leaves an error of order e^3
+__device__ __forceinline__ double rsq_h3(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+// orders a wavefront's own LDS writes before its later reads
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
-// FILT: the image-path loader drops the sources beyond reach of the chunk (above); it
-// pays where bins are dense (a 20% packing: 10% less time) and costs where they are
-// sparse (a tube with ~8 sources per fine bin: 6% more), so the host chooses it by the
-// mean number of sources per fine bin.
-template <bool SL, bool DL, bool FILT>
-__global__ void __launch_bounds__(PT *PW) __attribute__((amdgpu_waves_per_eu(6))) k_pair(PairArgs a) {
+// SL: single-layer term present (c1 != 0); DL: double-layer term present (c2 != 0).
+//
+// A wavefront takes one cluster of PC = 8 neighbouring targets of a fine bin at a time
+// (lane = 8 slot + target).  It streams the candidate sources of the rows of bins in reach
+// 64 at a time, one per lane, keeps those within rc of the cluster's bounding sphere, packs
+// their records back to back in its own LDS stage, and evaluates the stage eight sources by
+// eight targets per step; the slots' sums are added by shuffles at the end.  The work is
+// bound by FP64 issue (about 50 instructions a pair) and by the latency of a step's chain
+// (record, distance, table entry), so what matters is how many lanes of a step hold a pair
+// within rc and how many wavefronts run: 64 targets sharing a source filled 43% of the
+// lanes of the steps that had any (the chunk is as wide as a fine bin) and paid a step for
+// the candidates that paired with none; eight targets in Z order, which span a third of a
+// bin, fill 56% of all steps.  The sixteen wavefronts of the one workgroup per compute unit
+// share an LDS copy of the double-layer table: a step gathers 64 unrelated entries, which
+// the LDS serves in about 8 cycles per 32 lanes and the vector cache in 64 or more.  Both
+// layers together read their tables from memory and take twelve wavefronts (153 registers).
+// Measured, 512 cells at 20% (296k targets, 7.3e8 pairs, double layer): 5.76 ms with 64
+// targets per source, 3.66 so; 128 cells, 20,011 free points, both layers: 1.31 -> 0.75.
+// Two targets a lane (half the record reads, twelve wavefronts): 4.2 ms; the densities read
+// from memory instead of the stage: 4.1; 16 targets a cluster: 4.9.
+// The clusters are handed out by tickets, so uneven clusters do not leave a unit idle;
+// each cluster's sums do not depend on who takes it.
+//
+// Periodic images: the reference takes the minimum image of every candidate,
+// d - NINT(d / Lb) Lb.  When every dimension has at least 2R+3 fine bins, the image of
+// an in-cutoff pair is fixed by the bin walk: the source bin's wrap count k_run, the
+// target's box index kt (targets may lie outside [0, Lb)) and the source's (zero for a
+// source inside the box) give d = fl(xs - xi) + fl((k_run + kt) Lb), the same two
+// roundings as the reference's fl(fl(xs - xi) - fl(NINT * Lb)) with NINT = -(k_run +
+// kt); a candidate whose image differs is farther than rc either way.  Runs of one wrap
+// count are streamed together; a batch holding a source outside the box takes the
+// reference's formula.
+template <bool SL, bool DL>
+__global__ void __launch_bounds__(64 * (SL ? 12 : 16)) k_pair(PairArgs a) {
+  constexpr int PNW = SL ? 12 : 16;      // wavefronts (both layers need more registers)
   constexpr int NP = (SL ? 3 : 0) + (DL ? 6 : 0);
-  constexpr int PD = SL ? 3 : 0;  // first DL payload slot
+  constexpr int PD = SL ? 3 : 0;         // first DL payload value
+  constexpr bool LT = DL && !SL;         // the one table fits beside the stages
+  __shared__ double ltab[LT ? RBC_NTAB + 2 : 1];
+  constexpr int N2 = 2 + (NP + 1) / 2;   // 16-byte words of a record: x, y, z, node + 1, densities
+  __shared__ double2 stage[PNW][PCAP * N2];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int nb = a.nfbins, ncl = a.clus_off[nb] - a.clus_off[0];
+  // each XCD starts on its own contiguous range of clusters, whose sources then stay in
+  // its L2, and helps the others when that is done
+  const int xcd = (int)(blockIdx.x % RBC_NXCD), per = (ncl + RBC_NXCD - 1) / RBC_NXCD;
+  auto range = [&](int r) -> int { return max(0, min(per, ncl - r * per)); };
+  auto blocks = [&](int r) -> int { return ((int)gridDim.x - r + RBC_NXCD - 1) / RBC_NXCD; };
+  if ((int)(blockIdx.x / RBC_NXCD) >= range(xcd)) return;
+  if (LT) {
+    for (int t = threadIdx.x; t < RBC_NTAB + 2; t += 64 * PNW) ltab[t] = a.dl1[t];
+    __syncthreads();
+  }
+  const int tsub = lane & (PC - 1), slot = lane / PC;
+  const int Nf0 = a.Nf[0], Nf1 = a.Nf[1], Nf2 = a.Nf[2];
+  const double L0 = a.Lb[0], L1 = a.Lb[1], L2 = a.Lb[2];
+  const double iL0 = a.iLb[0], iL1 = a.iLb[1], iL2 = a.iLb[2];
+  const size_t np = a.np;
+  // pair statistics: the count, and sum (ti + 1)(node + 1) modulo 2^64
+  unsigned long long npairs = 0, csum = 0;
+
+  // the first cluster of every wavefront is fixed (one per compute unit first), the rest
+  // come from the ranges' tickets
+  int rg = xcd, k0 = wv * blocks(xcd) + (int)(blockIdx.x / RBC_NXCD);
+  int tried = 0;
+  // (few clusters: every range is covered by its workgroups' first ones, and the tickets,
+  // which cost a trip to memory each, stay untouched)
+  const bool tickets = per > PNW * (int)(gridDim.x / RBC_NXCD);
+  while (true) {
+    if (!tickets && k0 >= range(xcd)) break;
+    while (k0 >= range(rg) && tried < RBC_NXCD) {  // the next range that has clusters left
+      if (++tried == RBC_NXCD) break;
+      rg = rg + 1 == RBC_NXCD ? 0 : rg + 1;
+      int t = 0;
+      if (lane == 0) t = atomicAdd(a.ticket + rg, 1) + PNW * blocks(rg);
+      k0 = __builtin_amdgcn_readfirstlane(t);
+    }
+    if (tried == RBC_NXCD) break;
+    const int cl = rg * per + k0;
+    int next = ncl;
+    if (tickets && lane == 0) next = atomicAdd(a.ticket + rg, 1) + PNW * blocks(rg);
+    const int2 cb = a.clus[cl];
+    const int bin = cb.x, tend = a.tbin_start[bin + 1];
+    const int b1 = bin % Nf0, b2 = (bin / Nf0) % Nf1, b3 = bin / (Nf0 * Nf1);
+    const int k = cb.y + tsub;
+    const int ti = k < tend ? a.torder[k] : 0;
+    const bool act = k < tend && a.tact[ti] != 0;
+    if (__ballot(act) != 0ull) {
+      const double xi0 = a.tx[ti], xi1 = a.tx[ti + (size_t)a.nT], xi2 = a.tx[ti + 2 * (size_t)a.nT];
+      // the target's box index per dimension, by the binning's own arithmetic (k_bins):
+      // unwrapped bin = wrapped bin + kt Nf
+      const int kt0 = ((int)floor(xi0 * a.iLbNf[0]) - b1) / Nf0,
+                kt1 = ((int)floor(xi1 * a.iLbNf[1]) - b2) / Nf1,
+                kt2 = ((int)floor(xi2 * a.iLbNf[2]) - b3) / Nf2;
+      // the target's cell: its nodes are [off, off + npt), and 1 - the mask of its
+      // node q is maskcat[moff + ((q - base) mod npt)]
+      int off1 = 0, base1 = 0, moff = 0;  // (of node + 1)
+      unsigned npt = 0;
+      const int surf_i = act ? a.tindx[ti] : 0;
+      if (surf_i >= 1 && surf_i <= a.nrbc) {
+        const CellRec &cr = a.cells[surf_i - 1];
+        const int ilat_i = a.tindx[ti + a.nT] - 1, ilon_i = a.tindx[ti + 2 * (size_t)a.nT] - 1;
+        off1 = cr.off + 1;
+        npt = (unsigned)(cr.nlat * cr.nlon);
+        base1 = cr.off + 1 + ilon_i * cr.nlat;
+        moff = a.maskoff[cr.gtype] + ilat_i * (int)npt;
+      }
+      // The cluster's bounding sphere over its active targets, each taken back into the
+      // box (x - kt Lb): a candidate whose image (or minimum image) is farther than
+      // rc + r (plus a margin far above the roundings) from the centre is beyond rc of
+      // every target.  All slots hold the same targets.
+      double ct0, ct1, ct2, cut;
+      {
+        const double w0 = act ? xi0 - kt0 * L0 : 0., w1 = act ? xi1 - kt1 * L1 : 0.,
+                     w2 = act ? xi2 - kt2 * L2 : 0.;
+        double s0 = w0, s1 = w1, s2 = w2, n = act ? 1. : 0.;
+#pragma unroll
+        for (int o = PC / 2; o > 0; o >>= 1) {
+          s0 += __shfl_xor(s0, o, 64);
+          s1 += __shfl_xor(s1, o, 64);
+          s2 += __shfl_xor(s2, o, 64);
+          n += __shfl_xor(n, o, 64);
+        }
+        ct0 = s0 / n;
+        ct1 = s1 / n;
+        ct2 = s2 / n;
+        double r2 = act ? (w0 - ct0) * (w0 - ct0) + (w1 - ct1) * (w1 - ct1) + (w2 - ct2) * (w2 - ct2)
+                        : 0.;
+#pragma unroll
+        for (int o = PC / 2; o > 0; o >>= 1) r2 = fmax(r2, __shfl_xor(r2, o, 64));
+        cut = wave_uniform(a.rc * (1. + 1e-9) + sqrt(r2) + 1e-9 * (1. + L0 + L1 + L2));
+        ct0 = wave_uniform(ct0);
+        ct1 = wave_uniform(ct1);
+        ct2 = wave_uniform(ct2);
+      }
+      const double cut2 = wave_uniform(cut * cut);
+      double acc0 = 0, acc1 = 0, acc2 = 0;
+      unsigned long long nsum = 0;
+      unsigned cnt = 0;
+      bool mimg = false;                    // the stage takes minimum images (else the shift)
+      bool shift = false;                   // some target's shift is not zero
+      double sh0 = 0, sh1 = 0, sh2 = 0;     // image shift of the staged sources
+      int staged = 0;
+      double2 *st = stage[wv];
+
+      // Evaluates the staged sources [0, n) (n a multiple of PQ) against the targets, PQ at a
+      // time; lanes without a pair within rc run along and add nothing.  MODE 0: no image
+      // shift, 1: the target's shift, 2: minimum images.
+      auto eval = [&](auto mode, int n) {
+        constexpr int MODE = decltype(mode)::value;
+        const double2 *r = st + N2 * slot;
+#pragma unroll 1
+        for (int b = 0; b < n; b += PQ, r += N2 * PQ) {
+          const double2 p01 = r[0], p2m = r[1];
+          double pay[NP + 2];
+#pragma unroll
+          for (int q = 0; q < (NP + 1) / 2; q++) {
+            const double2 v = r[2 + q];
+            pay[2 * q] = v.x;
+            pay[2 * q + 1] = v.y;
+          }
+          const int node1 = __double2loint(p2m.y);
+          // 1 - mask for sources on the target's own cell: asked for first, used at the end
+          double cw = 1.;
+          if (NP > 0) {
+            const bool same = (unsigned)(node1 - off1) < npt;
+            if (__builtin_amdgcn_ballot_w64(same) != 0ull) {
+              int q = node1 - base1;
+              q += q < 0 ? (int)npt : 0;
+              if (same) cw = a.maskcat[moff + q];
+            }
+          }
+          double d0, d1, d2, s2;
+          {
+#pragma clang fp contract(off)
+            d0 = p01.x - xi0;
+            d1 = p01.y - xi1;
+            d2 = p2m.x - xi2;
+            if (MODE == 1) {
+              d0 = d0 + sh0;
+              d1 = d1 + sh1;
+              d2 = d2 + sh2;
+            } else if (MODE == 2) {
+              // rint differs from NINT only at |x/Lb| = 1/2, where |x| = Lb/2 > rc
+              d0 = d0 - rint(d0 * iL0) * L0;
+              d1 = d1 - rint(d1 * iL1) * L1;
+              d2 = d2 - rint(d2 * iL2) * L2;
+            }
+            const double t = d0 * d0 + d1 * d1;
+            s2 = t + d2 * d2;
+          }
+          // sqrt(s2) <= rc is certain below rc^2 (1 - 1e-12); in the thin shell above, the
+          // correctly rounded square root decides, as in the reference.  Below r_eps, and
+          // past the table's end, the coefficients are zero.
+          bool in = s2 < a.rc2lo;
+          if (__builtin_amdgcn_ballot_w64((!in && s2 <= a.rc2hi) || s2 < a.reps2) != 0ull) {
+            if (!in && s2 <= a.rc2hi) {
+              const double rr = sqrt(s2);
+              in = rr <= a.rc;
+              if (rr * a.tabscale >= (double)RBC_NTAB) cw = 0.;
+            } else if (s2 < a.reps2) {
+              s2 = a.reps2;
+              cw = 0.;
+            }
+          }
+          in = in && act;
+          cnt += (unsigned)__popcll(__builtin_amdgcn_ballot_w64(in));
+          double ir = 0, c1 = 0, c2 = 0, c3 = 0;
+          if (NP > 0) {
+            ir = rsq_h3(s2);
+            const double s = s2 * ir * a.tabscale, tf = __builtin_amdgcn_fract(s);
+            const int i = min((int)s, RBC_NTAB);  // (lanes beyond rc: any entry)
+            auto lerp = [&](const double *t) {
+              const double t0 = t[i], t1 = t[i + 1];
+              return fma(tf, t1 - t0, t0);
+            };
+            if (SL) {
+              c1 = lerp(a.sl1);
+              c2 = lerp(a.sl2);
+            }
+            if (DL) c3 = lerp(LT ? ltab : a.dl1);
+          }
+          const double ir2 = ir * ir;
+          double v0 = 0, v1 = 0, v2 = 0, cc = 0;
+          if (SL) {
+            const double EA = c1 * ir * ir2 + c2 * ir2, EB = c1 * ir - c2;
+            const double f0 = pay[0], f1 = pay[1], f2 = pay[2];
+            const double xf = EA * (d0 * f0 + d1 * f1 + d2 * f2), c = cw * a.c1;
+            v0 = c * (xf * d0 + EB * f0);
+            v1 = c * (xf * d1 + EB * f1);
+            v2 = c * (xf * d2 + EB * f2);
+          }
+          if (DL) {
+            const double EA = c3 * (ir2 * ir2 * ir);
+            const double xg = d0 * pay[PD] + d1 * pay[PD + 1] + d2 * pay[PD + 2];
+            const double xn = d0 * pay[PD + 3] + d1 * pay[PD + 4] + d2 * pay[PD + 5];
+            cc = (SL ? cw * a.c2 : cw) * EA * xg * xn;
+          }
+          if (in) {
+            asm volatile("");  // a masked update, not a select of its result
+            nsum += (unsigned)node1;
+            if (SL) {
+              acc0 += v0;
+              acc1 += v1;
+              acc2 += v2;
+            }
+            if (DL) {
+              acc0 += cc * d0;
+              acc1 += cc * d1;
+              acc2 += cc * d2;
+            }
+          }
+        }
+      };
+      for (int rb = 0; rb < a.nrows; rb += 32) {
+        // An x-row of source bins is one or two runs of sorted sources (a range shorter
+        // than the row wraps at most once), each with its wrap counts.  Lane 32 h + r holds
+        // run h of row rb + r.
+        const int row = rb + (lane & 31), h = lane >> 5;
+        int r_s = 0, r_n = 0, r_c = 0;
+        if (row < a.nrows) {
+          const unsigned code = (unsigned)a.rows[row];
+          int alo = (int)(code & 255) - 128, ahi = (int)((code >> 8) & 255) - 128;
+          const int o2 = (int)((code >> 16) & 255) - 128, o3 = (int)(code >> 24) - 128;
+          const int y = b2 + o2, z = b3 + o3;
+          if (a.img) {
+            // only the bins that the sphere of radius cut about the centre reaches
+            const double dy = fmax(0., fmax(y * a.w[1] - ct1, ct1 - (y + 1) * a.w[1])),
+                         dz = fmax(0., fmax(z * a.w[2] - ct2, ct2 - (z + 1) * a.w[2]));
+            const double h2 = cut2 - dy * dy - dz * dz;
+            if (h2 < 0.) {
+              ahi = alo - 1;
+            } else {
+              const double h = sqrt(h2) + 1e-9 * L0;
+              alo = max(alo, (int)floor((ct0 - h) * a.iLbNf[0]) - b1);
+              ahi = min(ahi, (int)floor((ct0 + h) * a.iLbNf[0]) - b1);
+            }
+          }
+          if (alo <= ahi) {
+            const int rowbase = Nf0 * (imod_d(y, Nf1) + Nf1 * imod_d(z, Nf2));
+            const int kyz = a.img ? (((y < 0 ? -1 : (y >= Nf1 ? 1 : 0)) + 1) << 2) |
+                                        (((z < 0 ? -1 : (z >= Nf2 ? 1 : 0)) + 1) << 4)
+                                  : 0;
+            int rlo[2] = {0, 0}, rhi[2] = {0, 0}, kx[2] = {0, 0}, nrun = 1;
+            if (ahi - alo + 1 >= Nf0) {
+              rlo[0] = 0;
+              rhi[0] = Nf0 - 1;
+            } else {
+              const int x0 = b1 + alo, x1 = b1 + ahi;
+              if (x0 >= Nf0) {
+                rlo[0] = x0 - Nf0, rhi[0] = x1 - Nf0, kx[0] = 1;
+              } else if (x1 < 0) {
+                rlo[0] = x0 + Nf0, rhi[0] = x1 + Nf0, kx[0] = -1;
+              } else if (x0 < 0) {
+                rlo[0] = x0 + Nf0, rhi[0] = Nf0 - 1, rlo[1] = 0, rhi[1] = x1, nrun = 2;
+                kx[0] = -1;
+              } else if (x1 >= Nf0) {
+                rlo[0] = x0, rhi[0] = Nf0 - 1, rlo[1] = 0, rhi[1] = x1 - Nf0, nrun = 2;
+                kx[1] = 1;
+              } else {
+                rlo[0] = x0, rhi[0] = x1;
+              }
+            }
+            if (h < nrun) {
+              r_s = a.bin_start[rowbase + (h ? rlo[1] : rlo[0])];
+              r_n = a.bin_start[rowbase + (h ? rhi[1] : rhi[0]) + 1] - r_s;
+              r_c = a.img ? ((h ? kx[1] : kx[0]) + 1) | kyz : 0;
+            }
+          }
+        }
+        {
+          unsigned long long rem = __ballot(r_n > 0);
+          while (rem) {  // the runs of one wrap count at a time
+            const int gcode = __builtin_amdgcn_readlane(r_c, __ffsll((long long)rem) - 1);
+            const unsigned long long grp = __ballot(r_n > 0 && r_c == gcode);
+            rem &= ~grp;
+            double e0, e1, e2;  // source + e: its image relative to the centre
+            {
+              const int k0 = (gcode & 3) - 1, k1 = ((gcode >> 2) & 3) - 1, k2 = ((gcode >> 4) & 3) - 1;
+              sh0 = (double)(k0 + kt0) * L0;
+              sh1 = (double)(k1 + kt1) * L1;
+              sh2 = (double)(k2 + kt2) * L2;
+              shift = __ballot(sh0 != 0. || sh1 != 0. || sh2 != 0.) != 0ull;
+              e0 = wave_uniform((double)k0 * L0 - ct0);
+              e1 = wave_uniform((double)k1 * L1 - ct1);
+              e2 = wave_uniform((double)k2 * L2 - ct2);
+            }
+            // inclusive prefix of the group's run lengths over the lanes
+            const int gn = (grp >> lane) & 1 ? r_n : 0;
+            int inc = gn;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+              const int u = __shfl_up(inc, o, 64);
+              if (lane >= o) inc += u;
+            }
+            const int total = __builtin_amdgcn_readlane(inc, 63);
+            // long runs are walked one by one; short ones (sparse bins) are packed back to
+            // back into full batches, each lane finding its source's run by bisection
+            const bool pack = total < 48 * __popcll(grp);
+            const int adj = r_s - (inc - gn);
+            unsigned long long runs = grp;
+            int pos = 0, end = 0;
+            if (pack) end = total;
+            int q = -1, node = 0;
+            double x0 = 0, x1 = 0, x2 = 0;
+            auto fetch = [&]() -> bool {
+              if (pos >= end && !pack && runs) {
+                const int r = __ffsll((long long)runs) - 1;
+                runs &= runs - 1;
+                pos = __builtin_amdgcn_readlane(r_s, r);
+                end = pos + __builtin_amdgcn_readlane(r_n, r);
+              }
+              q = -1;
+              if (pos >= end) return false;
+              const int g = pos + lane;
+              pos += 64;
+              int qq = g;
+              if (pack) {
+                int lo = 0;
+#pragma unroll
+                for (int s = 32; s > 0; s >>= 1)
+                  if (__shfl(inc, lo + s - 1, 64) <= g) lo += s;
+                qq = g + __shfl(adj, lo & 63, 64);
+              }
+              if (g < end) {
+                q = qq;
+                x0 = a.rec[qq];
+                x1 = a.rec[qq + np];
+                x2 = a.rec[qq + 2 * np];
+                node = a.src_node[qq];
+              }
+              return true;
+            };
+            bool more = fetch();
+#pragma unroll 1
+            while (more || staged > 0) {
+              const bool hv = more && q >= 0;
+              const bool m = !a.img || __ballot(hv && node < 0) != 0ull;
+              // the stage is emptied before the formula changes and at the end of the group
+              const bool drain = !more || (m != mimg && staged > 0);
+              if (!drain) {
+                mimg = m;
+                double g0, g1, g2;
+                if (m) {
+                  g0 = x0 - ct0;
+                  g1 = x1 - ct1;
+                  g2 = x2 - ct2;
+                  g0 -= rint(g0 * iL0) * L0;
+                  g1 -= rint(g1 * iL1) * L1;
+                  g2 -= rint(g2 * iL2) * L2;
+                } else {
+                  g0 = x0 + e0;
+                  g1 = x1 + e1;
+                  g2 = x2 + e2;
+                }
+                const bool keep = hv && g0 * g0 + g1 * g1 + g2 * g2 <= cut2;
+                const unsigned long long bk = __ballot(keep);
+                if (keep) {
+                  double2 *r = st + (staged + __popcll(bk & ((1ull << lane) - 1ull))) * N2;
+                  r[0] = make_double2(x0, x1);
+                  r[1] = make_double2(x2, __hiloint2double(0, (node & 0x7fffffff) + 1));
+                  const double2 *gf = (const double2 *)(a.rec + SREC_F(np) + 4 * (size_t)q),
+                                *gg = (const double2 *)(a.rec + SREC_G(np) + 6 * (size_t)q);
+                  if (SL) {
+                    const double2 u0 = gf[0], u1 = gf[1], v0 = gg[0], v1 = gg[1], v2 = gg[2];
+                    r[2] = u0;
+                    r[3] = make_double2(u1.x, v0.x);
+                    r[4] = make_double2(v0.y, v1.x);
+                    r[5] = make_double2(v1.y, v2.x);
+                    r[6] = make_double2(v2.y, 0.);
+                  } else if (DL) {
+                    const double2 v0 = gg[0], v1 = gg[1], v2 = gg[2];
+                    r[2] = v0;
+                    r[3] = v1;
+                    r[4] = v2;
+                  }
+                }
+                staged += __popcll(bk);
+                more = fetch();  // in flight while the stage is evaluated
+              }
+              int n = staged & ~(PQ - 1);
+              if (drain && n < staged) {
+                // fill the last step with sources beyond every target's reach (no comparison
+                // with an infinite or undefined square holds)
+                if (lane < n + PQ - staged) st[(staged + lane) * N2] = make_double2(__builtin_inf(), 0.);
+                n += PQ;
+              }
+              wave_lds_fence();
+              if (n == 0) continue;
+              if (mimg)
+                eval(std::integral_constant<int, 2>(), n);
+              else if (shift)
+                eval(std::integral_constant<int, 1>(), n);
+              else
+                eval(std::integral_constant<int, 0>(), n);
+              // the few left over move to the front
+              staged = max(staged - n, 0);
+              if (lane < staged * N2) {
+                const double2 v = st[n * N2 + lane];
+                st[lane] = v;
+              }
+              wave_lds_fence();
+            }
+          }
+        }
+      }
+      npairs += cnt;
+      // the slots' sums, in a fixed order
+#pragma unroll
+      for (int o = PC; o < 64; o <<= 1) {
+        acc0 += __shfl_xor(acc0, o, 64);
+        acc1 += __shfl_xor(acc1, o, 64);
+        acc2 += __shfl_xor(acc2, o, 64);
+      }
+      if (slot == 0 && act) {
+        const double f = (SL ? 1. : a.c2) / a.tA[ti];
+        a.vpair[ti] = f * acc0;
+        a.vpair[ti + (size_t)a.nT] = f * acc1;
+        a.vpair[ti + 2 * (size_t)a.nT] = f * acc2;
+      }
+      csum += (unsigned long long)(ti + 1) * nsum;
+    }
+    k0 = __builtin_amdgcn_readfirstlane(next);
+  }
+  // one atomic per wavefront for the pair statistics
+  for (int o = 32; o > 0; o >>= 1) csum += __shfl_xor(csum, o, 64);
+  if (lane == 0 && npairs) {
+    atomicAdd(&a.stat[0], npairs);
+    atomicAdd(&a.stat[1], csum);
+  }
+}
+
+// The single layer alone (the cells' right-hand side).  One workgroup takes 64 targets of a
+// fine bin, which its four wavefronts hold in common while they split every 256-source tile
+// between them; the partial sums are added in wavefront order.  Its two tables do not fit
+// the LDS beside the stages of k_pair, and the summation order of a sparse packing feeds a
+// wall solve whose iteration count follows the last bits, so it keeps the order of the
+// sources in the bins.  FILT: the loader drops the sources beyond reach of the chunk's
+// bounding sphere; it pays where bins are dense (a 20% packing: 10% less time) and costs
+// where they are sparse (a tube with ~8 sources per fine bin: 6% more), so the host chooses
+// it by the mean number of sources per fine bin.
+template <bool FILT>
+__global__ void __launch_bounds__(PT *PW) __attribute__((amdgpu_waves_per_eu(6))) k_pair_sl(PairArgs a) {
   __shared__ double sx[PS], sy[PS], sz[PS];
-  __shared__ double sp[NP > 0 ? NP : 1][PS];
+  __shared__ double sp[3][PS];
   __shared__ int snode[PS], scell[PS], sll[PS];
   __shared__ double red[PW - 1][3][PT];
   __shared__ int wout[PW], wkeep[PW];  // per wavefront: a source outside the box; sources kept
@@ -596,8 +1129,8 @@ __global__ void __launch_bounds__(PT *PW) __attribute__((amdgpu_waves_per_eu(6))
   const bool have = k < t1;
   const int ti = have ? a.torder[k] : 0;
   const bool act = have && a.tact[ti] != 0;
-  double xi0 = 0, xi1 = 0, xi2 = 0, cA1 = 0, cA2 = 0;
-  int ilon_i = 0, nn_i = 1, cell_i = -1;
+  double xi0 = 0, xi1 = 0, xi2 = 0, cA1 = 0;
+  int ilon_i = 0, nl_i = 1, nn_i = 1, cell_i = -1;
   const double *mtab = nullptr;  // the target's row of the same-surface mask table
   const int Nf0 = a.Nf[0], Nf1 = a.Nf[1], Nf2 = a.Nf[2];
   const int b1 = bin % Nf0, b2 = (bin / Nf0) % Nf1, b3 = bin / (Nf0 * Nf1);
@@ -612,11 +1145,11 @@ __global__ void __launch_bounds__(PT *PW) __attribute__((amdgpu_waves_per_eu(6))
     kt2 = ((int)floor(xi2 * a.iLbNf[2]) - b3) / Nf2;
     double Ai = a.tA[ti];
     cA1 = a.c1 / Ai;
-    cA2 = a.c2 / Ai;
     int surf_i = a.tindx[ti];
     if (surf_i >= 1 && surf_i <= a.nrbc) {
       const CellRec &cr = a.cells[surf_i - 1];
       cell_i = surf_i - 1;
+      nl_i = cr.nlat;
       nn_i = cr.nlon;
       const int ilat_i = a.tindx[ti + a.nT] - 1;
       mtab = a.mask[cr.gtype] + (size_t)ilat_i * cr.nlat * cr.nlon;
@@ -689,11 +1222,11 @@ __global__ void __launch_bounds__(PT *PW) __attribute__((amdgpu_waves_per_eu(6))
       const int jl = ll & 0xffff, jn = ll >> 16;
       int dl = jn - ilon_i;
       dl += dl < 0 ? nn_i : 0;
-      wm = 1. - mtab[jl * nn_i + dl];
+      wm = 1. - mtab[dl * nl_i + jl];
     }
     npairs++;
     nsum += (unsigned)(node + 1);
-    if (SL && ir != 0.) {
+    if (ir != 0.) {
       double EA, EB;
       ewald_sl_ir(a.sl1, a.sl2, rr, ir, a.tabscale, EA, EB);
       const double f0 = sp[0][j], f1 = sp[1][j], f2 = sp[2][j];
@@ -702,15 +1235,6 @@ __global__ void __launch_bounds__(PT *PW) __attribute__((amdgpu_waves_per_eu(6))
       acc0 += cc * (EA * d0 * xf + EB * f0);
       acc1 += cc * (EA * d1 * xf + EB * f1);
       acc2 += cc * (EA * d2 * xf + EB * f2);
-    }
-    if (DL && ir != 0.) {
-      const double EA = ewald_dl_ir(a.dl1, rr, ir, a.tabscale);
-      const double xg = d0 * sp[PD][j] + d1 * sp[PD + 1][j] + d2 * sp[PD + 2][j];
-      const double xn = d0 * sp[PD + 3][j] + d1 * sp[PD + 4][j] + d2 * sp[PD + 5][j];
-      const double cc = wm * cA2 * EA * xg * xn;
-      acc0 += cc * d0;
-      acc1 += cc * d1;
-      acc2 += cc * d2;
     }
   };
 
@@ -752,16 +1276,14 @@ __global__ void __launch_bounds__(PT *PW) __attribute__((amdgpu_waves_per_eu(6))
         const bool hv = t < cnt;
         const int q = base + t;
         double x0 = 0., x1 = 0., x2 = 0.;
+        int node = 0;
         bool out = false, keep = hv;
         if (hv) {
           x0 = a.rec[q];
           x1 = a.rec[q + np];
           x2 = a.rec[q + 2 * np];
-          if (a.img) {
-            const double f0 = floor(x0 * a.iLbNf[0]), f1 = floor(x1 * a.iLbNf[1]),
-                         f2 = floor(x2 * a.iLbNf[2]);
-            out = f0 < 0 || f0 >= Nf0 || f1 < 0 || f1 >= Nf1 || f2 < 0 || f2 >= Nf2;
-          }
+          node = a.src_node[q];
+          out = a.img && node < 0;
           if (FILT && a.img) {
             const double e0 = x0 + rsh0 - ct0, e1 = x1 + rsh1 - ct1, e2 = x2 + rsh2 - ct2;
             keep = e0 * e0 + e1 * e1 + e2 * e2 <= cut2;
@@ -791,16 +1313,8 @@ __global__ void __launch_bounds__(PT *PW) __attribute__((amdgpu_waves_per_eu(6))
           sx[pos] = x0;
           sy[pos] = x1;
           sz[pos] = x2;
-          if (SL)
-            for (int d = 0; d < 3; d++) sp[d][pos] = a.rec[q + np * (3 + d)];
-          if (DL) {
-            const double Bj = a.rec[q + np * 12];
-            for (int d = 0; d < 3; d++) {
-              sp[PD + d][pos] = a.rec[q + np * (6 + d)] * Bj;
-              sp[PD + 3 + d][pos] = a.rec[q + np * (9 + d)];
-            }
-          }
-          snode[pos] = a.src_node[q];
+          for (int d = 0; d < 3; d++) sp[d][pos] = a.rec[SREC_F(np) + 4 * (size_t)q + d];
+          snode[pos] = node & 0x7fffffff;
           scell[pos] = a.src_node[q + np];
           sll[pos] = a.src_node[q + 2 * np];
         }
@@ -1124,15 +1638,14 @@ __global__ void __launch_bounds__(PT *PW) k_pair32(Pair32Args a) {
               sph[t] = h;
               spl[t] = l;
               if (SL)
-                sfv[t] = make_float4((float)a.rec[q + np * 3], (float)a.rec[q + np * 4],
-                                     (float)a.rec[q + np * 5], 0.f);
+              {
+                const double *f = a.rec + SREC_F(np) + 4 * (size_t)q;
+                sfv[t] = make_float4((float)f[0], (float)f[1], (float)f[2], 0.f);
+              }
               if (DL) {
-                const double Bj = a.rec[q + np * 12];
-                sgn[2 * t] = make_float4((float)(a.rec[q + np * 6] * Bj),
-                                         (float)(a.rec[q + np * 7] * Bj),
-                                         (float)(a.rec[q + np * 8] * Bj), (float)a.rec[q + np * 9]);
-                sgn[2 * t + 1] = make_float4((float)a.rec[q + np * 10], (float)a.rec[q + np * 11],
-                                             0.f, 0.f);
+                const double *g = a.rec + SREC_G(np) + 6 * (size_t)q;
+                sgn[2 * t] = make_float4((float)g[0], (float)g[1], (float)g[2], (float)g[3]);
+                sgn[2 * t + 1] = make_float4((float)g[4], (float)g[5], 0.f, 0.f);
               }
             } else {
               sph[t] = make_float4(1e30f, 1e30f, 1e30f, __int_as_float(-2));
@@ -1168,7 +1681,7 @@ __global__ void __launch_bounds__(PT *PW) k_pair32(Pair32Args a) {
                 const int ll = __float_as_int(pl.w);
                 int dl = (ll >> 16) - ilon_i;
                 dl += dl < 0 ? nn_i : 0;
-                wm = 1.f - mtab[((size_t)ilat_i * nl_i + (ll & 0xffff)) * nn_i + dl];
+                wm = 1.f - mtab[((size_t)ilat_i * nn_i + dl) * nl_i + (ll & 0xffff)];
               }
               const float ir2 = ir * ir;
               if (SL) {
@@ -1213,7 +1726,7 @@ __global__ void __launch_bounds__(PT *PW) k_pair32(Pair32Args a) {
                 const int ll = __float_as_int(pl.w);
                 int dl = (ll >> 16) - ilon_i;
                 dl += dl < 0 ? nn_i : 0;
-                wm = 1. - mtabd[((size_t)ilat_i * nl_i + (ll & 0xffff)) * nn_i + dl];
+                wm = 1. - mtabd[((size_t)ilat_i * nn_i + dl) * nl_i + (ll & 0xffff)];
               }
               if (SL) {
                 double EA, EB;
@@ -1939,6 +2452,26 @@ int rbc_type_ptrs(rbc3d_ctx *c, TypePtrs *tp) {
     for (size_t i = 0; i < nt; i++) pf[i] = c->gtypes[i]->d_maskf.p;
     RBC_TRY(c->d_tp_maskf.ensure(nt));
     HIP_TRY(hipMemcpy(c->d_tp_maskf.p, pf.data(), nt * sizeof(pf[0]), hipMemcpyHostToDevice));
+    // 1 - the same-surface masks back to back, with their offsets
+    std::vector<int> mo(nt);
+    size_t mtot = 0;
+    for (size_t i = 0; i < nt; i++) {
+      mo[i] = (int)mtot;
+      mtot += c->gtypes[i]->d_mask.n;
+    }
+    if (mtot >= (1ull << 31)) {
+      rbc_set_error("same-surface mask tables too large");
+      return RBC3D_EINVAL;
+    }
+    RBC_TRY(c->d_maskcat.ensure(mtot));
+    RBC_TRY(c->d_maskoff.ensure(nt));
+    std::vector<double> mc(mtot);
+    for (size_t i = 0; i < nt; i++)
+      HIP_TRY(hipMemcpy(mc.data() + mo[i], c->gtypes[i]->d_mask.p,
+                        c->gtypes[i]->d_mask.n * sizeof(double), hipMemcpyDeviceToHost));
+    for (double &v : mc) v = 1. - v;
+    HIP_TRY(hipMemcpy(c->d_maskcat.p, mc.data(), mtot * sizeof(double), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(c->d_maskoff.p, mo.data(), nt * sizeof(int), hipMemcpyHostToDevice));
     RBC_TRY(c->d_tp_ptr.ensure(ptr.size()));
     RBC_TRY(c->d_tp_int.ensure(ni.size()));
     HIP_TRY(hipMemcpy(c->d_tp_ptr.p, ptr.data(), ptr.size() * sizeof(ptr[0]), hipMemcpyHostToDevice));
@@ -1967,15 +2500,15 @@ static int exclusive_scan(rbc3d_ctx *c, const int *in, int *out, int n) {
   return RBC3D_OK;
 }
 
-// launch the split-form pair kernel with the arguments of the FP64 one
-template <bool SL, bool DL>
-static void launch_pair(bool filt, int nblk, hipStream_t st, const PairArgs &pa) {
-  if (filt)
-    k_pair<SL, DL, true><<<nblk, PT * PW, 0, st>>>(pa);
+static void launch_pair_sl(rbc3d_ctx *c, int nblk, const PairArgs &pa) {
+  // the source filter where fine bins hold 32 sources or more on average
+  if (c->pair_img && c->np >= 32 * (long long)c->nfbins)
+    k_pair_sl<true><<<nblk, PT * PW, 0, c->stream>>>(pa);
   else
-    k_pair<SL, DL, false><<<nblk, PT * PW, 0, st>>>(pa);
+    k_pair_sl<false><<<nblk, PT * PW, 0, c->stream>>>(pa);
 }
 
+// launch the split-form pair kernel with the arguments of the FP64 one
 static int launch_pair32(rbc3d_ctx *c, const PairArgs &pa, int nblk_max,
                          const float *const *maskf) {
   Pair32Args a;
@@ -2069,34 +2602,55 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   cacheable = cacheable && c->geom_reuse;
   const bool hit = cacheable && c->cache_epoch == c->geom_epoch && c->cache_nT == nT;
   c->cache_epoch = -1;  // valid again only when this call completes as cacheable
-  RBC_TRY(c->d_flag.ensure(2 * (size_t)(nb + 1) + 8));
-  int *chunk_cnt = c->d_flag.p + 8, *chunk_off = chunk_cnt + (nb + 1);
+  // [0..7] flags, [8..15] the pair kernel's tickets, then the chunk and cluster counts
+  // per fine bin and their scan
+  RBC_TRY(c->d_flag.ensure(4 * (size_t)(nb + 1) + 16));
+  int *chunk_cnt = c->d_flag.p + 16, *chunk_off = chunk_cnt + 2 * (nb + 1);
+  const size_t ncl_max = (size_t)nT / PC + std::min(nb, nT) + 1;
   if (!hit) {
-    // targets binned like the sources
-    RBC_TRY(c->d_tbin.ensure(nT + 1));
+    // targets binned like the sources, in Z order inside a bin where the key fits
+    RBC_TRY(c->d_tbin.ensure(3 * (size_t)nT + 3));
     RBC_TRY(c->d_torder.ensure(nT + 1));
     RBC_TRY(c->d_tbin_start.ensure(nb + 1));
+    RBC_TRY(c->d_clus.ensure(2 * ncl_max));
+    int *kin = c->d_tbin.p, *kout = kin + nT + 1, *iin = kout + nT + 1;
+    const int sub = nb <= (1 << 24) ? 64 : 1;
+    int bits = 1;
+    while ((1LL << bits) < (long long)sub * nb) bits++;
     rbc_stage_begin(c, ST_TSORT);
-    RBC_TRY(fine_sort(c, nT, d_tx, nT, c->d_tbin.p, c->d_torder.p, c->d_tbin_start.p));
+    k_target_keys<<<(nT + 255) / 256, 256, 0, st>>>(nT, d_tx, fine_geom(c), sub, kin, iin);
+    size_t tmp = 0;
+    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, kin, kout, iin, c->d_torder.p, nT, 0,
+                                               bits, st));
+    RBC_TRY(c->d_cub_tmp.ensure(tmp + 16));
+    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->d_cub_tmp.p, tmp, kin, kout, iin, c->d_torder.p,
+                                               nT, 0, bits, st));
+    k_target_bin_start<<<(nb + 1 + 255) / 256, 256, 0, st>>>(nT, kout, nb, sub, c->d_tbin_start.p);
     rbc_stage_end(c, ST_TSORT);
     k_chunks<<<(nb + 1 + 255) / 256, 256, 0, st>>>(nb, c->d_tbin_start.p, chunk_cnt);
-    RBC_TRY(exclusive_scan(c, chunk_cnt, chunk_off, nb + 1));
+    RBC_TRY(exclusive_scan(c, chunk_cnt, chunk_off, 2 * (nb + 1)));
+    k_clusters<<<(nb + 255) / 256, 256, 0, st>>>(nb, c->d_tbin_start.p, chunk_off + nb + 1,
+                                                 (int2 *)c->d_clus.p);
+    HIP_TRY(hipGetLastError());
   }
   RBC_TRY(c->d_vacc.ensure((size_t)3 * nT + 1));
   RBC_TRY(c->d_pairstat.ensure(2));
   // cleared by kernels, not memsets: this path is recorded into graphs
   k_fill_u64<<<1, 64, 0, st>>>(c->d_pairstat.p, 2, 0ull);
-  k_fill_i<<<1, 64, 0, st>>>(c->d_flag.p, 8, 0);
+  k_fill_i<<<1, 64, 0, st>>>(c->d_flag.p, 16, 0);
   PairArgs pa;
   for (int d = 0; d < 3; d++) {
     pa.Lb[d] = c->Lb[d];
     pa.iLb[d] = c->iLb[d];
     pa.iLbNf[d] = c->iLbNf[d];
     pa.Nf[d] = c->Nf[d];
+    pa.w[d] = c->Lb[d] / c->Nf[d];
   }
   pa.img = c->pair_img;
   pa.rc = c->conf.rc;
+  pa.rc2 = c->conf.rc * c->conf.rc;
   pa.rc2hi = c->conf.rc * c->conf.rc * (1.0 + 1e-12);
+  pa.rc2w = c->conf.rc * c->conf.rc * 2e-12;
   pa.rc2lo = c->conf.rc * c->conf.rc * (1.0 - 1e-12);
   pa.reps2 = c->r_eps * c->r_eps;
   pa.tabscale = RBC_NTAB / c->conf.rc;
@@ -2111,13 +2665,13 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   pa.rec = c->d_src_rec.p;
   pa.src_node = c->d_work.p;
   pa.bin_start = c->d_fbin_start.p;
-  pa.node_cell = c->d_node_cell.p;
-  pa.node_ll = c->d_node_ll.p;
   pa.cells = c->d_cells.p;
   pa.sl1 = c->d_sl1.p;
   pa.sl2 = c->d_sl2.p;
   pa.dl1 = c->d_dl1.p;
   pa.mask = tp->mask;
+  pa.maskcat = c->d_maskcat.p;
+  pa.maskoff = c->d_maskoff.p;
   pa.tx = d_tx;
   pa.tA = d_A;
   pa.tindx = d_tindx;
@@ -2125,6 +2679,9 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   pa.torder = c->d_torder.p;
   pa.tbin_start = c->d_tbin_start.p;
   pa.chunk_off = chunk_off;
+  pa.clus_off = chunk_off + nb + 1;
+  pa.clus = (const int2 *)c->d_clus.p;
+  pa.ticket = c->d_flag.p + 8;
   pa.vpair = c->d_vacc.p;
   pa.stat = c->d_pairstat.p;
   int nblk = nb + (nT + PT - 1) / PT + 1;
@@ -2132,16 +2689,21 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   if (c->prec == RBC3D_PREC_SPLIT && c->split_pair32) {
     RBC_TRY(launch_pair32(c, pa, nblk, tp->maskf));
   } else {
-    // the source filter where fine bins hold 32 sources or more on average
-    const bool filt = c->pair_img && c->np >= 32 * (long long)nb;
-    if (c1 != 0 && c2 != 0)
-      launch_pair<true, true>(filt, nblk, st, pa);
+    // one workgroup per compute unit: its LDS holds the table and the wavefronts' stages
+    const unsigned grid = (unsigned)std::min<size_t>(c->ncu, ncl_max);
+    // cells of viscosity ratio 1 have no double layer (its density carries Bcoef = 0); the
+    // reciprocal part still takes it, so an undefined density shows in every velocity
+    bool dl = false;
+    for (const CellRec &r : c->cells) dl = dl || r.Bcoef != 0.;
+    dl = dl && c2 != 0;
+    if (c1 != 0 && dl)
+      k_pair<true, true><<<grid, 64 * 12, 0, st>>>(pa);
     else if (c1 != 0)
-      launch_pair<true, false>(filt, nblk, st, pa);
-    else if (c2 != 0)
-      launch_pair<false, true>(filt, nblk, st, pa);
+      launch_pair_sl(c, nblk, pa);
+    else if (dl)
+      k_pair<false, true><<<grid, 64 * 16, 0, st>>>(pa);
     else
-      launch_pair<false, false>(filt, nblk, st, pa);
+      k_pair<false, false><<<grid, 64 * 16, 0, st>>>(pa);
   }
   rbc_stage_end(c, ST_PAIR);
   HIP_TRY(hipGetLastError());
