@@ -15,8 +15,8 @@
 // 16 mt + 4 (l / 16) + i of output tile mt, which is exactly the B operand of K-step mt
 // of the next layer, so activations never leave the registers.  The backward pass
 // uses the same layout with W^T; the weight gradients dW = dZ^T H (k: nodes) take
-// both operands through an LDS transpose and accumulate in LDS, one workgroup of one
-// wavefront per partial sum, reduced over workgroups in a fixed order.
+// both operands through an LDS transpose and accumulate in registers; a workgroup's
+// wavefronts and then the workgroups are summed in a fixed order.
 #include <cmath>
 #include <vector>
 
@@ -46,7 +46,16 @@ enum { WB_1 = 0, WB_2 = WB_1 + 64 * 16, WB_3 = WB_2 + 64 * 64, WB_4 = WB_3 + 64 
 // 4 (1 x 4), then the biases b1 b2 b3 (64 each) and b4 (16, 3 used)
 enum { GA_1 = 0, GA_2 = GA_1 + 4 * 256, GA_3 = GA_2 + 16 * 256, GA_4 = GA_3 + 16 * 256,
        GA_B = GA_4 + 4 * 256, GA_N = GA_B + 3 * 64 + 16 };
-#define MLP_TS 72  // LDS row stride (bf16) of the transpose tiles: 64 + 8
+#define MLP_TS 72  // LDS row stride (bf16) of the transpose tiles and 64-wide weights: 64 + 8
+#define MLP_TS1 24 // of the 16-wide ones: 16 + 8
+// LDS copies of the weights with padded rows (16 rows of 128 bytes would share banks),
+// and of W2^T, W3^T, W4^T for the backward pass
+enum { SW_1 = 0, SW_2 = SW_1 + 64 * MLP_TS1, SW_3 = SW_2 + 64 * MLP_TS, SW_4 = SW_3 + 64 * MLP_TS,
+       SW_N = SW_4 + 16 * MLP_TS,
+       ST_2 = SW_N, ST_3 = ST_2 + 64 * MLP_TS, ST_4 = ST_3 + 64 * MLP_TS, ST_N = ST_4 + 64 * MLP_TS1 };
+#define MLP_TW 4   // wavefronts per training workgroup
+// LDS copies of the biases b1 b2 b3 (64 each), b4 (3) and the norm
+enum { SB_4 = 3 * 64, SB_NORM = SB_4 + 4, SB_N = SB_NORM + 2 * MLP_NIN + MLP_NOUT };
 
 struct rbc3d_mlp {
   hipStream_t stream = nullptr;  // own stream, or `ext` once rbc3d_mlp_set_stream was
@@ -67,45 +76,30 @@ __device__ __forceinline__ unsigned short f2bf(float f) {  // round to nearest e
 }
 __device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float((unsigned)h << 16); }
 
-// GELU, tanh form (Hendrycks and Gimpel, 2016), and its derivative
-#define GELU_C 0.7978845608028654f  // sqrt(2/pi)
+// GELU, tanh form (Hendrycks and Gimpel, 2016), and its derivative d.  With
+// u = sqrt(2/pi) (x + 0.044715 x^3) and (1 + tanh u) / 2 = s = 1 / (1 + exp(-2u)):
+// gelu = x s, d = s + x s (1 - s) 2 u'.  Seven instructions with the hardware's exponential
+// and reciprocal (one unit in the last place each); through tanh with its division it was
+// about thirty, which bound both kernels, and lost digits of 1 + tanh below zero.
+#define GELU_2C 1.5957691216057308f  // 2 sqrt(2/pi)
 #define GELU_A 0.044715f
-__device__ __forceinline__ float mlp_tanh(float u) {
-  const float e = __expf(2.f * u);
-  return 1.f - 2.f / (e + 1.f);
-}
-__device__ __forceinline__ float gelu(float x) {
-  const float t = mlp_tanh(GELU_C * (x + GELU_A * x * x * x));
-  return 0.5f * x * (1.f + t);
-}
-__device__ __forceinline__ float gelu_d(float x) {
-  const float t = mlp_tanh(GELU_C * (x + GELU_A * x * x * x));
-  return 0.5f * (1.f + t) + 0.5f * x * (1.f - t * t) * GELU_C * (1.f + 3.f * GELU_A * x * x);
+#define GELU_LOG2E 1.4426950408889634f
+__device__ __forceinline__ float gelu(float x, float &d) {
+  const float x2 = x * x;
+  const float e = x * fmaf(-GELU_2C * GELU_LOG2E * GELU_A, x2, -GELU_2C * GELU_LOG2E);
+  const float s = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(e)), g = x * s;
+  d = fmaf(g * (1.f - s), fmaf(3.f * GELU_2C * GELU_A, x2, GELU_2C), s);
+  return g;
 }
 
 __device__ __forceinline__ mlp_f4 mfma(mlp_s4 a, mlp_s4 b, mlp_f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-// A operand from a row-major BF16 matrix W[rows][ld]: lane supplies W[r0 + l%16][k0 + 4q + j]
+// A operand from a row-major BF16 matrix W[rows][ld] (8-byte aligned rows): lane supplies
+// W[r0 + l%16][k0 + 4q + j]
 __device__ __forceinline__ mlp_s4 ldA(const unsigned short *W, int ld, int r0, int k0, int lane) {
-  const unsigned short *p = W + (size_t)(r0 + (lane & 15)) * ld + k0 + 4 * (lane >> 4);
-  mlp_s4 a;
-  a[0] = (short)p[0];
-  a[1] = (short)p[1];
-  a[2] = (short)p[2];
-  a[3] = (short)p[3];
-  return a;
-}
-// A operand of W^T: lane supplies W^T[r0 + l%16][k0 + 4q + j] = W[k0 + 4q + j][r0 + l%16]
-__device__ __forceinline__ mlp_s4 ldAT(const unsigned short *W, int ld, int r0, int k0, int lane) {
-  const unsigned short *p = W + (size_t)(k0 + 4 * (lane >> 4)) * ld + r0 + (lane & 15);
-  mlp_s4 a;
-  a[0] = (short)p[0];
-  a[1] = (short)p[ld];
-  a[2] = (short)p[2 * ld];
-  a[3] = (short)p[3 * ld];
-  return a;
+  return *reinterpret_cast<const mlp_s4 *>(W + (r0 + (lane & 15)) * ld + k0 + 4 * (lane >> 4));
 }
 __device__ __forceinline__ mlp_s4 tobf(mlp_f4 v) {
   mlp_s4 r;
@@ -117,17 +111,18 @@ __device__ __forceinline__ mlp_s4 tobf(mlp_f4 v) {
 }
 
 // Forward pass of one tile of 16 nodes (node = node0 + lane % 16); keeps the
-// pre-activations z and the BF16 activations h (B-operand layout) for the backward.
+// activations' derivatives and the BF16 activations h (B-operand layout) for the backward.
 struct MlpTile {
   mlp_s4 x;         // inputs (features 4q + j)
-  mlp_f4 z[3][4];   // pre-activations of the hidden layers, tile mt
+  mlp_f4 d[3][4];   // GELU' at the hidden layers' pre-activations, tile mt
   mlp_s4 h[3][4];   // BF16 activations of the hidden layers, K-step mt
   mlp_f4 y;         // outputs 4q + i (valid: q == 0, i < 3)
 };
 
-__device__ __forceinline__ void mlp_forward(const unsigned short *sW, const float *p,
-                                            const float *norm, const float *X, int n, int node0,
-                                            int lane, MlpTile &T) {
+__device__ __forceinline__ void mlp_forward(const unsigned short *sW, const float *sb,
+                                            const float *X, int n, int node0, int lane,
+                                            MlpTile &T) {
+  const float *norm = sb + SB_NORM;
   const int q = lane >> 4, node = node0 + (lane & 15);
   #pragma unroll
   for (int j = 0; j < 4; j++) {
@@ -140,46 +135,78 @@ __device__ __forceinline__ void mlp_forward(const unsigned short *sW, const floa
   #pragma unroll
   for (int mt = 0; mt < 4; mt++) {
     mlp_f4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma(ldA(sW + WB_1, 16, 16 * mt, 0, lane), T.x, acc);
+    acc = mfma(ldA(sW + SW_1, MLP_TS1, 16 * mt, 0, lane), T.x, acc);
     #pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] += p[MP_B1 + 16 * mt + 4 * q + i];
-    T.z[0][mt] = acc;
+    for (int i = 0; i < 4; i++) acc[i] += sb[16 * mt + 4 * q + i];
     mlp_f4 g;
     #pragma unroll
-    for (int i = 0; i < 4; i++) g[i] = gelu(acc[i]);
+    for (int i = 0; i < 4; i++) {
+      float d;
+      g[i] = gelu(acc[i], d);
+      T.d[0][mt][i] = d;
+    }
     T.h[0][mt] = tobf(g);
   }
   // layers 2 and 3: 64 x 64
   #pragma unroll
   for (int L = 1; L < 3; L++) {
-    const unsigned short *W = sW + (L == 1 ? WB_2 : WB_3);
-    const float *b = p + (L == 1 ? MP_B2 : MP_B3);
+    const unsigned short *W = sW + (L == 1 ? SW_2 : SW_3);
+    const float *b = sb + 64 * L;
     #pragma unroll
     for (int mt = 0; mt < 4; mt++) {
       mlp_f4 acc = {0.f, 0.f, 0.f, 0.f};
       #pragma unroll
-      for (int kt = 0; kt < 4; kt++) acc = mfma(ldA(W, 64, 16 * mt, 16 * kt, lane), T.h[L - 1][kt], acc);
+      for (int kt = 0; kt < 4; kt++) acc = mfma(ldA(W, MLP_TS, 16 * mt, 16 * kt, lane), T.h[L - 1][kt], acc);
       #pragma unroll
       for (int i = 0; i < 4; i++) acc[i] += b[16 * mt + 4 * q + i];
-      T.z[L][mt] = acc;
       mlp_f4 g;
       #pragma unroll
-      for (int i = 0; i < 4; i++) g[i] = gelu(acc[i]);
+      for (int i = 0; i < 4; i++) {
+        float d;
+        g[i] = gelu(acc[i], d);
+        T.d[L][mt][i] = d;
+      }
       T.h[L][mt] = tobf(g);
     }
   }
   // layer 4: W4p[16][64]
   mlp_f4 acc = {0.f, 0.f, 0.f, 0.f};
   #pragma unroll
-  for (int kt = 0; kt < 4; kt++) acc = mfma(ldA(sW + WB_4, 64, 0, 16 * kt, lane), T.h[2][kt], acc);
+  for (int kt = 0; kt < 4; kt++) acc = mfma(ldA(sW + SW_4, MLP_TS, 0, 16 * kt, lane), T.h[2][kt], acc);
   #pragma unroll
-  for (int i = 0; i < 4; i++) acc[i] += (q == 0 && i < MLP_NOUT) ? p[MP_B4 + i] : 0.f;
+  for (int i = 0; i < 4; i++) acc[i] += (q == 0 && i < MLP_NOUT) ? sb[SB_4 + i] : 0.f;
   T.y = acc;
 }
 
-__device__ __forceinline__ void load_weights(unsigned short *sW, const unsigned short *wb) {
-  for (int t = threadIdx.x; t < WB_N / 4; t += blockDim.x)
-    reinterpret_cast<uint2 *>(sW)[t] = reinterpret_cast<const uint2 *>(wb)[t];
+// the biases and the norm, which every tile reads, into LDS
+__device__ __forceinline__ void load_biases(float *sb, const float *p, const float *norm) {
+  for (int t = threadIdx.x; t < SB_N; t += blockDim.x)
+    sb[t] = t < 64             ? p[MP_B1 + t]
+            : t < 128          ? p[MP_B2 + t - 64]
+            : t < SB_4         ? p[MP_B3 + t - 128]
+            : t < SB_4 + 3     ? p[MP_B4 + t - SB_4]
+            : t < SB_NORM      ? 0.f
+                               : norm[t - SB_NORM];
+}
+// the BF16 weights into their padded LDS layout (tr: the transposes too)
+__device__ __forceinline__ void load_weights(unsigned short *sW, const unsigned short *wb, bool tr) {
+  static_assert(WB_N % 4 == 0, "four weights at a time");
+  #pragma unroll 5
+  for (int t4 = threadIdx.x; t4 < WB_N / 4; t4 += 256) {
+    const mlp_s4 v = reinterpret_cast<const mlp_s4 *>(wb)[t4];
+    const int t = 4 * t4;
+    if (t < WB_2) {
+      *reinterpret_cast<mlp_s4 *>(sW + SW_1 + (t >> 4) * MLP_TS1 + (t & 15)) = v;
+    } else {
+      const int o = t - WB_2, r = o >> 6, k = o & 63;  // rows of W2, W3, W4
+      *reinterpret_cast<mlp_s4 *>(sW + SW_2 + r * MLP_TS + k) = v;
+      if (tr)
+        #pragma unroll
+        for (int j = 0; j < 4; j++)
+          sW[r < 128 ? ST_2 + ((r & 64) + k + j) * MLP_TS + (r & 63)
+                     : ST_4 + (k + j) * MLP_TS1 + r - 128] = (unsigned short)v[j];
+    }
+  }
 }
 
 // inference: Y[node][c] = scale_c * y_c (the predicted traction increment)
@@ -187,27 +214,27 @@ __global__ void __launch_bounds__(256) k_mlp_forward(int n, const float *__restr
                                                      const unsigned short *__restrict__ wb,
                                                      const float *__restrict__ p,
                                                      const float *__restrict__ norm, float *Y) {
-  __shared__ __align__(16) unsigned short sW[WB_N];
-  load_weights(sW, wb);
+  __shared__ __align__(16) unsigned short sW[SW_N];
+  __shared__ float sb[SB_N];
+  load_biases(sb, p, norm);
+  load_weights(sW, wb, false);
   __syncthreads();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int ntile = (n + 15) / 16, nw = gridDim.x * (blockDim.x >> 6);
   for (int tile = blockIdx.x * (blockDim.x >> 6) + wv; tile < ntile; tile += nw) {
     MlpTile T;
-    mlp_forward(sW, p, norm, X, n, 16 * tile, lane, T);
+    mlp_forward(sW, sb, X, n, 16 * tile, lane, T);
     const int node = 16 * tile + (lane & 15);
     if (lane < 16 && node < n)
       #pragma unroll
-      for (int i = 0; i < MLP_NOUT; i++) Y[(size_t)node * MLP_NOUT + i] = T.y[i] * norm[2 * MLP_NIN + i];
+      for (int i = 0; i < MLP_NOUT; i++) Y[(size_t)node * MLP_NOUT + i] = T.y[i] * sb[SB_NORM + 2 * MLP_NIN + i];
   }
 }
 
 // transpose tile: S[node][feature] in LDS, row stride MLP_TS
 __device__ __forceinline__ void st_tile(unsigned short *S, int f0, mlp_s4 v, int lane) {
   // lane holds node l%16, features f0 + 4q + j
-  unsigned short *r = S + (lane & 15) * MLP_TS + f0 + 4 * (lane >> 4);
-  #pragma unroll
-  for (int j = 0; j < 4; j++) r[j] = (unsigned short)v[j];
+  *reinterpret_cast<mlp_s4 *>(S + (lane & 15) * MLP_TS + f0 + 4 * (lane >> 4)) = v;
 }
 // operand from a transposed tile: lane supplies M[node 4q + j][c0 + l%16]
 __device__ __forceinline__ mlp_s4 ld_tile(const unsigned short *S, int c0, int lane) {
@@ -217,132 +244,181 @@ __device__ __forceinline__ mlp_s4 ld_tile(const unsigned short *S, int c0, int l
   for (int j = 0; j < 4; j++) v[j] = (short)r[j * MLP_TS];
   return v;
 }
-// dW tile (mt, nt) += dZ^T H over the 16 nodes of the tile, accumulated in LDS
-__device__ __forceinline__ void acc_dw(float *acc, const unsigned short *SZ, int z0,
-                                       const unsigned short *SH, int h0, int lane) {
-  float *t = acc + 16 * (4 * (lane >> 4)) + (lane & 15);
-  mlp_f4 c;
-  #pragma unroll
-  for (int i = 0; i < 4; i++) c[i] = t[16 * i];
-  c = mfma(ld_tile(SZ, z0, lane), ld_tile(SH, h0, lane), c);
-  #pragma unroll
-  for (int i = 0; i < 4; i++) t[16 * i] = c[i];
+// orders a wavefront's own LDS accesses
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-// bias gradient: sum over the 16 nodes held by the lanes of one quarter
-__device__ __forceinline__ void acc_db(float *db, int f0, mlp_f4 v, int lane) {
+// a wavefront's gradient sums: dW in MFMA output tiles, db per lane over its nodes
+struct MlpAcc {
+  mlp_f4 w1[4], w2[16], w3[16], w4[4], b[3][4], b4;
+};
+// dW tiles += dZ^T H over the 16 nodes of the tile held in the transpose tiles
+template <int NM, int NN>
+__device__ __forceinline__ void acc_dw(mlp_f4 *acc, const unsigned short *SZ,
+                                       const unsigned short *SH, int lane) {
+  mlp_s4 zf[NM], hf[NN];
   #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    float s = v[i];
-    for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 16);
-    v[i] = s;
-  }
+  for (int m = 0; m < NM; m++) zf[m] = ld_tile(SZ, 16 * m, lane);
+  #pragma unroll
+  for (int k = 0; k < NN; k++) hf[k] = ld_tile(SH, 16 * k, lane);
+  #pragma unroll
+  for (int m = 0; m < NM; m++)
+    #pragma unroll
+    for (int k = 0; k < NN; k++) acc[NN * m + k] = mfma(zf[m], hf[k], acc[NN * m + k]);
+}
+// the wavefront's sums added to (first: stored in) the workgroup's, in ga_slot's layout;
+// all of a group's old sums are read before the first new one is stored, since one after
+// the other every sum would wait for the LDS twice
+template <int N>
+__device__ __forceinline__ void put_tiles(float *red, const mlp_f4 *v, int lane, bool first) {
+  float *t = red + 16 * (4 * (lane >> 4)) + (lane & 15);
+  mlp_f4 o[N];
+  #pragma unroll
+  for (int m = 0; m < N; m++)
+    #pragma unroll
+    for (int i = 0; i < 4; i++) o[m][i] = first ? 0.f : t[256 * m + 16 * i];
+  #pragma unroll
+  for (int m = 0; m < N; m++)
+    #pragma unroll
+    for (int i = 0; i < 4; i++) t[256 * m + 16 * i] = o[m][i] + v[m][i];
+}
+__device__ __forceinline__ void put_bias(float *red, mlp_f4 v, int lane, bool first) {
+  float *t = red + 4 * (lane >> 4);
+  mlp_f4 o;
+  #pragma unroll
+  for (int i = 0; i < 4; i++) o[i] = first ? 0.f : t[i];
+  #pragma unroll
+  for (int i = 0; i < 4; i++)
+    for (int k = 1; k < 16; k <<= 1) v[i] += __shfl_xor(v[i], k, 16);
   if ((lane & 15) == 0)
     #pragma unroll
-    for (int i = 0; i < 4; i++) db[f0 + 4 * (lane >> 4) + i] += v[i];
+    for (int i = 0; i < 4; i++) t[i] = o[i] + v[i];
 }
 
-// training: loss and gradient partial sums of one workgroup (one wavefront) over the
-// tiles blockIdx.x, blockIdx.x + gridDim.x, ...; targets are raw increments T[n][3]
-__global__ void __launch_bounds__(64) k_mlp_train(int n, const float *__restrict__ X,
+// training: loss and gradient partial sums of one workgroup over the 16-node tiles its
+// MLP_TW wavefronts take in turn; targets are raw increments T[n][3].  A wavefront keeps
+// all its sums in registers (160 of them matrix accumulators, one wavefront a SIMD): in
+// LDS, where every tile's products were added before, a tile cost 640 more LDS accesses
+// and 200 lane exchanges for the biases.  65,536 rows: 135 -> 58 us.
+__global__ void __launch_bounds__(64 * MLP_TW, 1) k_mlp_train(int n, const float *__restrict__ X,
                                                   const float *__restrict__ Tg,
                                                   const unsigned short *__restrict__ wb,
                                                   const float *__restrict__ p,
                                                   const float *__restrict__ norm, float *part,
                                                   double *lpart) {
-  __shared__ __align__(16) unsigned short sW[WB_N];
-  __shared__ __align__(16) unsigned short SZ[16 * MLP_TS], SH[16 * MLP_TS];
-  __shared__ float acc[GA_N];
-  load_weights(sW, wb);
-  for (int t = threadIdx.x; t < GA_N; t += 64) acc[t] = 0.f;
+  __shared__ __align__(16) unsigned short sW[ST_N];
+  __shared__ __align__(16) unsigned short tz[MLP_TW][16 * MLP_TS], th[MLP_TW][16 * MLP_TS];
+  __shared__ float red[GA_N];
+  __shared__ double lred[MLP_TW];
+  __shared__ float sb[SB_N];
+  load_biases(sb, p, norm);
+  load_weights(sW, wb, true);
   __syncthreads();
-  const int lane = threadIdx.x, q = lane >> 4;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, q = lane >> 4;
+  unsigned short *SZ = tz[wv], *SH = th[wv];
   const int ntile = (n + 15) / 16;
   const float gs = 2.f / (3.f * (float)n);
   double lsum = 0.;
-  for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+  MlpAcc A;
+  const mlp_f4 zero = {0.f, 0.f, 0.f, 0.f};
+  #pragma unroll
+  for (int t = 0; t < 16; t++) A.w2[t] = A.w3[t] = zero;
+  #pragma unroll
+  for (int t = 0; t < 4; t++) A.w1[t] = A.w4[t] = A.b[0][t] = A.b[1][t] = A.b[2][t] = zero;
+  A.b4 = zero;
+  for (int tile = blockIdx.x * MLP_TW + wv; tile < ntile; tile += gridDim.x * MLP_TW) {
     MlpTile T;
-    mlp_forward(sW, p, norm, X, n, 16 * tile, lane, T);
+    mlp_forward(sW, sb, X, n, 16 * tile, lane, T);
     const int node = 16 * tile + (lane & 15);
     // dL/dy of the normalised outputs
-    mlp_f4 dy = {0.f, 0.f, 0.f, 0.f};
+    mlp_f4 dy = zero;
     if (q == 0 && node < n)
       #pragma unroll
       for (int i = 0; i < MLP_NOUT; i++) {
-        const float e = T.y[i] - Tg[(size_t)node * MLP_NOUT + i] / norm[2 * MLP_NIN + i];
+        const float e = T.y[i] - Tg[(size_t)node * MLP_NOUT + i] / sb[SB_NORM + 2 * MLP_NIN + i];
         lsum += (double)e * e;
         dy[i] = gs * e;
       }
     const mlp_s4 dyb = tobf(dy);
     // layer 4: db4, dW4 = dY^T H3, dH3 = W4^T dY
-    acc_db(acc + GA_B + 192, 0, dy, lane);
+    A.b4 += dy;
+    wave_fence();
     st_tile(SZ, 0, dyb, lane);
     #pragma unroll
     for (int kt = 0; kt < 4; kt++) st_tile(SH, 16 * kt, T.h[2][kt], lane);
-    __syncthreads();
-    #pragma unroll
-    for (int nt = 0; nt < 4; nt++) acc_dw(acc + GA_4 + 256 * nt, SZ, 0, SH, 16 * nt, lane);
+    wave_fence();
+    acc_dw<1, 4>(A.w4, SZ, SH, lane);
     mlp_f4 dz[4];
     mlp_s4 dzb[4];
     #pragma unroll
     for (int mt = 0; mt < 4; mt++) {
-      mlp_f4 d = {0.f, 0.f, 0.f, 0.f};
-      d = mfma(ldAT(sW + WB_4, 64, 16 * mt, 0, lane), dyb, d);
-      #pragma unroll
-      for (int i = 0; i < 4; i++) d[i] *= gelu_d(T.z[2][mt][i]);
+      mlp_f4 d = mfma(ldA(sW + ST_4, MLP_TS1, 16 * mt, 0, lane), dyb, zero);
+      d *= T.d[2][mt];
       dz[mt] = d;
       dzb[mt] = tobf(d);
     }
     // layers 3 and 2: db, dW = dZ^T H_prev, dH_prev = W^T dZ
     #pragma unroll
     for (int L = 2; L >= 1; L--) {
-      const unsigned short *W = sW + (L == 2 ? WB_3 : WB_2);
-      float *dW = acc + (L == 2 ? GA_3 : GA_2);
-      #pragma unroll
-      for (int mt = 0; mt < 4; mt++) acc_db(acc + GA_B + 64 * L, 16 * mt, dz[mt], lane);
-      __syncthreads();
+      const unsigned short *WT = sW + (L == 2 ? ST_3 : ST_2);
+      wave_fence();
       #pragma unroll
       for (int mt = 0; mt < 4; mt++) {
+        A.b[L][mt] += dz[mt];
         st_tile(SZ, 16 * mt, dzb[mt], lane);
         st_tile(SH, 16 * mt, T.h[L - 1][mt], lane);
       }
-      __syncthreads();
-      for (int mt = 0; mt < 4; mt++)
-        #pragma unroll
-        for (int nt = 0; nt < 4; nt++) acc_dw(dW + 256 * (4 * mt + nt), SZ, 16 * mt, SH, 16 * nt, lane);
-      mlp_f4 nz[4];
+      wave_fence();
+      acc_dw<4, 4>(L == 2 ? A.w3 : A.w2, SZ, SH, lane);
       mlp_s4 nzb[4];
       #pragma unroll
       for (int mt = 0; mt < 4; mt++) {
-        mlp_f4 d = {0.f, 0.f, 0.f, 0.f};
+        mlp_f4 d = zero;
         #pragma unroll
-        for (int kt = 0; kt < 4; kt++) d = mfma(ldAT(W, 64, 16 * mt, 16 * kt, lane), dzb[kt], d);
-        #pragma unroll
-        for (int i = 0; i < 4; i++) d[i] *= gelu_d(T.z[L - 1][mt][i]);
-        nz[mt] = d;
+        for (int kt = 0; kt < 4; kt++) d = mfma(ldA(WT, MLP_TS, 16 * mt, 16 * kt, lane), dzb[kt], d);
+        d *= T.d[L - 1][mt];
+        dz[mt] = d;
         nzb[mt] = tobf(d);
       }
       #pragma unroll
-      for (int mt = 0; mt < 4; mt++) {
-        dz[mt] = nz[mt];
-        dzb[mt] = nzb[mt];
-      }
+      for (int mt = 0; mt < 4; mt++) dzb[mt] = nzb[mt];
     }
     // layer 1: db1, dW1 = dZ1^T X
+    wave_fence();
     #pragma unroll
-    for (int mt = 0; mt < 4; mt++) acc_db(acc + GA_B, 16 * mt, dz[mt], lane);
-    __syncthreads();
-    #pragma unroll
-    for (int mt = 0; mt < 4; mt++) st_tile(SZ, 16 * mt, dzb[mt], lane);
+    for (int mt = 0; mt < 4; mt++) {
+      A.b[0][mt] += dz[mt];
+      st_tile(SZ, 16 * mt, dzb[mt], lane);
+    }
     st_tile(SH, 0, T.x, lane);
-    __syncthreads();
-    #pragma unroll
-    for (int mt = 0; mt < 4; mt++) acc_dw(acc + GA_1 + 256 * mt, SZ, 16 * mt, SH, 0, lane);
-    __syncthreads();
+    wave_fence();
+    acc_dw<4, 1>(A.w1, SZ, SH, lane);
   }
   for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
-  __syncthreads();
-  for (int t = threadIdx.x; t < GA_N; t += 64) part[(size_t)blockIdx.x * GA_N + t] = acc[t];
-  if (lane == 0) lpart[blockIdx.x] = lsum;
+  if (lane == 0) lred[wv] = lsum;
+  for (int w = 0; w < MLP_TW; w++) {
+    if (w == wv) {
+      const bool first = w == 0;
+      put_tiles<4>(red + GA_1, A.w1, lane, first);
+      put_tiles<16>(red + GA_2, A.w2, lane, first);
+      put_tiles<16>(red + GA_3, A.w3, lane, first);
+      put_tiles<4>(red + GA_4, A.w4, lane, first);
+      #pragma unroll
+      for (int L = 0; L < 3; L++)
+        #pragma unroll
+        for (int t = 0; t < 4; t++) put_bias(red + GA_B + 64 * L + 16 * t, A.b[L][t], lane, first);
+      put_bias(red + GA_B + 192, A.b4, lane, first);
+    }
+    __syncthreads();
+  }
+  for (int t = threadIdx.x; t < GA_N; t += 64 * MLP_TW) part[(size_t)blockIdx.x * GA_N + t] = red[t];
+  if (threadIdx.x == 0) {
+    double s = 0.;
+    for (int w = 0; w < MLP_TW; w++) s += lred[w];
+    lpart[blockIdx.x] = s;
+  }
 }
 
 // accumulator slot of parameter p (the inverse of the tile layout above)
@@ -366,14 +442,25 @@ __device__ __forceinline__ int ga_slot(int p) {
   return GA_B + 192 + (p - MP_B4);
 }
 
-// grad[p] = sum over workgroups of the partials, in workgroup order
-__global__ void k_mlp_reduce(int nwg, const float *__restrict__ part, float *grad) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= MP_N) return;
-  const int s = ga_slot(p);
+// grad[p] = sum over workgroups of the partials: a workgroup takes 64 parameters, each of
+// its MLP_RW wavefronts the partials w, w + MLP_RW, ... in order, then the wavefronts in
+// order.  (One thread a parameter walked all partials one after the other: 131 us at 512
+// partials against 6 us at 256.)
+#define MLP_RW 16
+__global__ void __launch_bounds__(64 * MLP_RW) k_mlp_reduce(int nwg, const float *__restrict__ part,
+                                                            float *grad) {
+  __shared__ float red[MLP_RW][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, p = blockIdx.x * 64 + lane;
+  const int s = p < MP_N ? ga_slot(p) : 0;
   float g = 0.f;
-  for (int w = 0; w < nwg; w++) g += part[(size_t)w * GA_N + s];
-  grad[p] = g;
+  #pragma unroll 4
+  for (int w = wv; w < nwg; w += MLP_RW) g += part[(size_t)w * GA_N + s];
+  red[wv][lane] = g;
+  __syncthreads();
+  if (wv == 0 && p < MP_N) {
+    for (int w = 1; w < MLP_RW; w++) g += red[w][lane];
+    grad[p] = g;
+  }
 }
 
 // BF16 copy of the weights in the padded tile layout
@@ -515,12 +602,12 @@ extern "C" int rbc3d_mlp_forward_dev(rbc3d_mlp *m, int n, const float *d_x, floa
 static int mlp_grad(rbc3d_mlp *m, int n, const float *d_x, const float *d_t, double *loss) {
   hipStream_t st = m->st();
   const int ntile = (n + 15) / 16;
-  const int nwg = std::min(512, ntile);
+  const int nwg = std::min(256, (ntile + MLP_TW - 1) / MLP_TW);
   RBC_TRY(m->part.ensure((size_t)nwg * GA_N));
   RBC_TRY(m->lpart.ensure(nwg));
-  k_mlp_train<<<nwg, 64, 0, m->st()>>>(n, d_x, d_t, m->wb.p, m->p.p, m->norm.p, m->part.p,
-                                         m->lpart.p);
-  k_mlp_reduce<<<(MP_N + 255) / 256, 256, 0, m->st()>>>(nwg, m->part.p, m->grad.p);
+  k_mlp_train<<<nwg, 64 * MLP_TW, 0, m->st()>>>(n, d_x, d_t, m->wb.p, m->p.p, m->norm.p,
+                                                m->part.p, m->lpart.p);
+  k_mlp_reduce<<<(MP_N + 63) / 64, 64 * MLP_RW, 0, m->st()>>>(nwg, m->part.p, m->grad.p);
   HIP_TRY(hipGetLastError());
   if (loss) {
     std::vector<double> lp(nwg);
