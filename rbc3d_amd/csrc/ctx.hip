@@ -241,6 +241,28 @@ static int make_gtype(rbc3d_ctx *c, int nlat, GridType **out) {
   RBC_TRY(upload(g->d_thG, thG, st));
   RBC_TRY(upload(g->d_phiG, phiG, st));
   RBC_TRY(upload(g->d_pwt, wL, st));
+  {
+    // latitude rows of the patches: a row's points lie on the spline rows floor(th / h) and
+    // the next, the same for every longitude (spline_interp's own arithmetic)
+    const size_t npt = (size_t)nr * na;
+    std::vector<double> ps(thG.size());
+    std::vector<int> lo(nl), hi(nl);
+    const double hx = RBC_TWO_PI / (2 * nl), ihx = 1. / hx;
+    for (int ilat = 0; ilat < nl; ilat++) {
+      lo[ilat] = 1 << 20;
+      hi[ilat] = -1;
+      for (size_t q = 0; q < npt; q++) {
+        const int i1 = (int)floor(thG[npt * ilat + q] * ihx);
+        lo[ilat] = std::min(lo[ilat], i1);
+        hi[ilat] = std::max(hi[ilat], i1 + 1);
+        for (int j = 0; j < nn; j++)
+          ps[(npt * ilat + q) * nn + j] = phiG[npt * (ilat + (size_t)nl * j) + q];
+      }
+      g->nband = std::max(g->nband, hi[ilat] - lo[ilat] + 1);
+    }
+    RBC_TRY(upload(g->d_phiS, ps, st));
+    RBC_TRY(upload(g->d_band, lo, st));
+  }
   // same-surface mask MaskFunc(DistOnSphere/radius) by (ilat_i, ilon_j - ilon_i, ilat_j):
   // a row is the order of a cell's nodes, shifted to the target's longitude
   std::vector<double> mk((size_t)nl * nl * nn);
@@ -700,6 +722,7 @@ extern "C" int rbc3d_set_cells(rbc3d_ctx *c, int nrbc, const int *nlat0, const i
   HIP_TRY(hipMemsetAsync(c->d_gs.p, 0, sizeof(double) * 3 * np, st));
   HIP_TRY(hipMemsetAsync(c->d_spl.p, 0, sizeof(double) * (spl + 1), st));
   RBC_TRY(rbc_sh_build_splines(c, 0));  // x, a3, detJ splines
+  RBC_TRY(rbc_self_rows(c));
   RBC_TRY(rbc_build_source_list(c));
   HIP_TRY(hipStreamSynchronize(st));
   return RBC3D_OK;

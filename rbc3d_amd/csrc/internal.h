@@ -85,6 +85,11 @@ struct GridType {
   DBuf<double> d_Dm;     // periodic derivative matrix, length 2 nlat, [p][q]
   DBuf<double> d_Dn;     // periodic derivative matrix, length nlon, [p][q]
   DBuf<double> d_thG, d_phiG, d_pwt;  // polar patch: [node][irad + nrad*iazm], weights
+  // the patches of one latitude row: longitudes [ilat][point][ilon], and the band of nband
+  // spline rows their points fall in, starting at d_band[ilat]
+  DBuf<double> d_phiS;
+  DBuf<int> d_band;
+  int nband = 0;
   DBuf<double> d_mask;   // same-surface mask [ilat_i][dlon][ilat_j]
   DBuf<float> d_maskf;   // the same in FP32
   DBuf<double> d_proj;   // projection tables (RBC_PJ_*)
@@ -267,6 +272,11 @@ struct rbc3d_ctx {
   DBuf<int> d_maskoff;     // where each starts
   DBuf<const float *> d_tp_maskf;  // FP32 mask table per grid type
   DBuf<int> d_tp_int;
+  DBuf<const int *> d_tp_band;
+  // the self patch by latitude rows: (cell, ilat) list, LDS bytes (0: does not fit)
+  DBuf<int> d_self_rows;
+  int self_nrow = 0;
+  size_t self_lds = 0;
   size_t tp_ntypes = 0;
   StageTimer timer;
   // persistent cell-BIE solution (KSPSetInitialGuessNonzero, common/ModVelSolver.F90:87)
@@ -552,14 +562,16 @@ int rbc_sh_anal_batch(int nlat, int nlon, int nt, const double *d_g, int idg, in
 int rbc_sh_synth_batch(int nlat, int nlon, int nt, double *d_g, int idg, int jdg, const double *d_a,
                        const double *d_b, int ida, int jda, int equi, hipStream_t st);
 int rbc_build_source_list(rbc3d_ctx *c);
+int rbc_self_rows(rbc3d_ctx *c);  // launch list of the self patches by latitude rows
 // device arrays of per-grid-type table pointers, indexed by CellRec::gtype (pair.hip):
 // same-surface mask, grid colatitudes and longitudes, patch points and weights, projection
 // tables (patch directions and least-squares weights)
 struct TypePtrs {
   const double *const *mask, *const *th, *const *phi, *const *thG, *const *phiG, *const *pwt,
-      *const *proj;
+      *const *proj, *const *phiS;
+  const int *const *band;
   const float *const *maskf;
-  const int *nrad, *nazm;
+  const int *nrad, *nazm, *nband;
 };
 int rbc_type_ptrs(rbc3d_ctx *c, TypePtrs *tp);
 int rbc_update_density(rbc3d_ctx *c, int which);

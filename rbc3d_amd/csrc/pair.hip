@@ -22,6 +22,9 @@
 #include "surf_core.h"
 
 #define NBR_T 256
+#define SELF_T 1024  // threads of a self-patch row workgroup
+#define SELF_VAR 9   // its spline variables: x, a3, g detJ
+#define SELF_PSTR (4 * SELF_VAR + 2)  // doubles of a spline point, two of padding: LDS banks
 
 // ---------------------------------------------------------------------------
 // cell list
@@ -460,6 +463,29 @@ __global__ void k_coarse_coords(int np, const double *__restrict__ x, HashGeom h
   int i1, i2, i3;
   hash_index3(xp, hg.Nc, hg.iLbNc, i1, i2, i3);
   cc[p] = (i1 - 1) | ((i2 - 1) << 10) | ((i3 - 1) << 20);
+}
+
+// The latitude rows of every cell for k_self_own, and its LDS size: the largest band among
+// the cells' grids; 0 where one does not fit (the general kernel then runs)
+int rbc_self_rows(rbc3d_ctx *c) {
+  size_t lds = sizeof(double) * 3 * SELF_T;  // at least the sums
+  std::vector<int> rl;
+  for (int i = 0; i < c->nrbc; i++) {
+    const CellRec &r = c->cells[i];
+    const GridType *g = c->gtypes[r.gtype];
+    lds = std::max(lds, sizeof(double) * SELF_PSTR * g->nband * g->nlon);
+    if (g->nlon > SELF_T) lds = SIZE_MAX / 2;
+    for (int k = 0; k < r.nlat; k++) {
+      rl.push_back(i);
+      rl.push_back(k);
+    }
+  }
+  c->self_lds = lds <= (size_t)c->lds_max ? lds : 0;
+  c->self_nrow = (int)(rl.size() / 2);
+  RBC_TRY(c->d_self_rows.ensure(rl.size() + 2));
+  if (!rl.empty())
+    HIP_TRY(hipMemcpy(c->d_self_rows.p, rl.data(), rl.size() * sizeof(int), hipMemcpyHostToDevice));
+  return RBC3D_OK;
 }
 
 int rbc_build_source_list(rbc3d_ctx *c) {
@@ -2113,6 +2139,111 @@ __global__ void __launch_bounds__(256) k_self(SingArgs a) {
   }
 }
 
+// RBC_SingInt of the double layer alone at the cells' own nodes (the cell matvec): one
+// workgroup per latitude row of a cell.  The patches of a row's targets reach a band of
+// nrows spline rows, which the workgroup copies into LDS once (nine variables; a point's
+// are together, PSTR doubles apart); thread (group, ilon) takes every ngrp-th patch point
+// of target ilon, and the groups are added in order.  The evaluation is bound by the bytes
+// of its 36 corner values a point (1152): from the vector cache at 64 bytes a cycle k_self
+// ran at its limit, the LDS gives twice that, and a target's lanes no longer compute 36
+// addresses.  The spline arithmetic is spline_interp's, operation for operation.
+// 512 cells of 17 x 34: 2.11 -> 1.21 ms; 4,096 cells of two grids: 10.6 -> 6.5.
+struct SelfArgs {
+  int nT;
+  double rc, reps, c2;
+  const CellRec *cells;
+  const int2 *rowlist;  // workgroup -> (cell, ilat)
+  const double *spl, *dl1;
+  const double *const *th, *const *phi, *const *thG, *const *phiS, *const *pwt;
+  const int *const *rows;  // per grid type: first spline row of each latitude's band
+  const int *nrad, *nazm, *nband;
+  double *dvself;
+};
+__global__ void __launch_bounds__(SELF_T) k_self_own(SelfArgs a) {
+  extern __shared__ __align__(16) double sband[];
+  const int2 rl = a.rowlist[blockIdx.x];
+  const CellRec cr = a.cells[rl.x];
+  const int gt = cr.gtype, m = 2 * cr.nlat, n = cr.nlon, ilat = rl.y;
+  const int npt = a.nrad[gt] * a.nazm[gt], nrad = a.nrad[gt], nb = a.nband[gt], r0 = a.rows[gt][ilat];
+  const double *blk = a.spl + cr.spl;
+  const size_t vs = (size_t)m * n * 4;
+  // the band: row r0 + i at i, all longitudes
+  for (int t = threadIdx.x; t < SELF_VAR * nb * n; t += SELF_T) {
+    const int i = t % nb, q = t / nb, j = q % n, v = q / n;
+    const int var = v < 3 ? SPL_X + v : v < 6 ? SPL_A3 + v - 3 : SPL_G + v - 6;
+    const int row = r0 + i < m ? r0 + i : r0 + i - m;
+    const double4 u = *(const double4 *)(blk + vs * var + 4 * (size_t)(row + m * j));
+    double *d = sband + (size_t)SELF_PSTR * (i + nb * j) + 4 * v;
+    *(double2 *)d = make_double2(u.x, u.y);
+    *(double2 *)(d + 2) = make_double2(u.z, u.w);
+  }
+  const int ngrp = SELF_T / n, grp = (int)threadIdx.x / n, ilon = (int)threadIdx.x - grp * n;
+  const bool live = grp < ngrp;
+  double dv0 = 0, dv1 = 0, dv2 = 0, xi[3] = {0, 0, 0};
+  if (live) spline_interp(blk + vs * SPL_X, m, n, a.th[gt][ilat], a.phi[gt][ilon], 3, xi);
+  __syncthreads();
+  if (live) {
+    const double *thG = a.thG[gt] + (size_t)npt * ilat;              // the same at every longitude
+    const double *phiS = a.phiS[gt] + (size_t)npt * n * ilat + ilon;  // [point][ilon]
+    const double *pw = a.pwt[gt];
+    const double hx = RBC_TWO_PI / m, hy = RBC_TWO_PI / n, ihx = 1. / hx, ihy = 1. / hy;
+    for (int p = grp; p < npt; p += ngrp) {
+      double f[SELF_VAR];
+      {
+        // spline_interp on the band, without FMA contraction
+#pragma clang fp contract(off)
+        const double x = thG[p], y = phiS[(size_t)n * p];
+        const double fi1 = floor(x * ihx), fj1 = floor(y * ihy);
+        const double s = x * ihx - fi1, t = y * ihy - fj1;
+        const int i1 = min(max((int)fi1 - r0, 0), nb - 2), i2 = i1 + 1;
+        const int j1 = wrap_idx((int)fj1, n), j2 = j1 + 1 == n ? 0 : j1 + 1;
+        const double cx0 = 1 + s * s * (-3. + 2. * s), cx1 = s * s * (3. - 2. * s);
+        const double cx2 = hx * s * (1. + s * (-2. + s)), cx3 = hx * s * s * (-1. + s);
+        const double cy0 = 1 + t * t * (-3. + 2. * t), cy1 = t * t * (3. - 2. * t);
+        const double cy2 = hy * t * (1. + t * (-2. + t)), cy3 = hy * t * t * (-1. + t);
+        const double2 *b11 = (const double2 *)(sband + (size_t)SELF_PSTR * (i1 + nb * j1)),
+                      *b12 = (const double2 *)(sband + (size_t)SELF_PSTR * (i1 + nb * j2)),
+                      *b21 = (const double2 *)(sband + (size_t)SELF_PSTR * (i2 + nb * j1)),
+                      *b22 = (const double2 *)(sband + (size_t)SELF_PSTR * (i2 + nb * j2));
+#pragma unroll 3
+        for (int l = 0; l < SELF_VAR; l++) {
+          const double2 a11 = b11[2 * l], c11 = b11[2 * l + 1], a12 = b12[2 * l], c12 = b12[2 * l + 1];
+          const double2 a21 = b21[2 * l], c21 = b21[2 * l + 1], a22 = b22[2 * l], c22 = b22[2 * l + 1];
+          const double q0 = a11.x * cy0 + a12.x * cy1 + c11.x * cy2 + c12.x * cy3;
+          const double q1 = a21.x * cy0 + a22.x * cy1 + c21.x * cy2 + c22.x * cy3;
+          const double q2 = a11.y * cy0 + a12.y * cy1 + c11.y * cy2 + c12.y * cy3;
+          const double q3 = a21.y * cy0 + a22.y * cy1 + c21.y * cy2 + c22.y * cy3;
+          f[l] = cx0 * q0 + cx1 * q1 + cx2 * q2 + cx3 * q3;
+        }
+      }
+      const double x0 = f[0] - xi[0], x1 = f[1] - xi[1], x2 = f[2] - xi[2];
+      const double rr = sqrt(x0 * x0 + x1 * x1 + x2 * x2);
+      if (rr >= a.rc) continue;
+      const double EA = ewald_dl(a.dl1, rr, a.reps, a.rc);
+      const double xg = x0 * f[6] + x1 * f[7] + x2 * f[8], xn = x0 * f[3] + x1 * f[4] + x2 * f[5];
+      const double w = pw[p % nrad] * (EA * xg * xn);
+      dv0 += w * x0;
+      dv1 += w * x1;
+      dv2 += w * x2;
+    }
+  }
+  __syncthreads();  // the band is consumed: its space takes the groups' sums
+  double(*red)[SELF_T] = reinterpret_cast<double(*)[SELF_T]>(sband);
+  red[0][threadIdx.x] = dv0;
+  red[1][threadIdx.x] = dv1;
+  red[2][threadIdx.x] = dv2;
+  __syncthreads();
+  if ((int)threadIdx.x < n) {
+    const double c2m = a.c2 * cr.Bcoef;
+    const int ti = cr.off + ilat + cr.nlat * (int)threadIdx.x;
+    for (int d = 0; d < 3; d++) {
+      double v = red[d][threadIdx.x];
+      for (int g = 1; g < ngrp; g++) v += red[d][g * n + threadIdx.x];
+      a.dvself[ti + (size_t)a.nT * d] = c2m != 0 ? c2m * v : 0.;
+    }
+  }
+}
+
 // Near-singular stage 1: translate the target next to the closest node, project it
 // onto the neighbour's spline surface (Spline_FindProjection) and apply the distance
 // test of RBC_NearSingInt.  One lane per (target, neighbouring cell) item; items are
@@ -2396,12 +2527,18 @@ __global__ void __launch_bounds__(256) k_linear_partial(int np, const double *__
     for (int d = 0; d < 3; d++) part[3 * blockIdx.x + d] = red[d][0];
 }
 
-__global__ void k_linear_final(int nb, const double *part, double scale, double *xv) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// the blocks' sums, by one wavefront (lanes stride the blocks, then a shuffle tree: one
+// thread walking 256 blocks took 27 us, this 4)
+__global__ void __launch_bounds__(64) k_linear_final(int nb, const double *part, double scale,
+                                                     double *xv) {
+  const int lane = threadIdx.x;
   double s[3] = {0, 0, 0};
-  for (int b = 0; b < nb; b++)
+  for (int b = lane; b < nb; b += 64)
     for (int d = 0; d < 3; d++) s[d] += part[3 * b + d];
-  for (int d = 0; d < 3; d++) xv[d] = scale * s[d];
+  for (int d = 0; d < 3; d++) {
+    s[d] = wave_sum(s[d]);
+    if (lane == 0) xv[d] = scale * s[d];
+  }
 }
 
 struct CombineArgs {
@@ -2434,8 +2571,9 @@ __global__ void k_combine(CombineArgs a) {
 int rbc_type_ptrs(rbc3d_ctx *c, TypePtrs *tp) {
   size_t nt = c->gtypes.size();
   if (c->tp_ntypes != nt) {
-    std::vector<const double *> ptr(7 * nt);
-    std::vector<int> ni(2 * nt);
+    std::vector<const double *> ptr(8 * nt);
+    std::vector<const int *> pb(nt);
+    std::vector<int> ni(3 * nt);
     for (size_t i = 0; i < nt; i++) {
       GridType *g = c->gtypes[i];
       ptr[0 * nt + i] = g->d_mask.p;
@@ -2445,6 +2583,9 @@ int rbc_type_ptrs(rbc3d_ctx *c, TypePtrs *tp) {
       ptr[4 * nt + i] = g->d_phiG.p;
       ptr[5 * nt + i] = g->d_pwt.p;
       ptr[6 * nt + i] = g->d_proj.p;
+      ptr[7 * nt + i] = g->d_phiS.p;
+      pb[i] = g->d_band.p;
+      ni[2 * nt + i] = g->nband;
       ni[i] = g->nrad;
       ni[nt + i] = g->nazm;
     }
@@ -2472,6 +2613,8 @@ int rbc_type_ptrs(rbc3d_ctx *c, TypePtrs *tp) {
     for (double &v : mc) v = 1. - v;
     HIP_TRY(hipMemcpy(c->d_maskcat.p, mc.data(), mtot * sizeof(double), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(c->d_maskoff.p, mo.data(), nt * sizeof(int), hipMemcpyHostToDevice));
+    RBC_TRY(c->d_tp_band.ensure(nt));
+    HIP_TRY(hipMemcpy(c->d_tp_band.p, pb.data(), nt * sizeof(pb[0]), hipMemcpyHostToDevice));
     RBC_TRY(c->d_tp_ptr.ensure(ptr.size()));
     RBC_TRY(c->d_tp_int.ensure(ni.size()));
     HIP_TRY(hipMemcpy(c->d_tp_ptr.p, ptr.data(), ptr.size() * sizeof(ptr[0]), hipMemcpyHostToDevice));
@@ -2486,9 +2629,12 @@ int rbc_type_ptrs(rbc3d_ctx *c, TypePtrs *tp) {
   tp->phiG = p + 4 * nt;
   tp->pwt = p + 5 * nt;
   tp->proj = p + 6 * nt;
+  tp->phiS = p + 7 * nt;
+  tp->band = c->d_tp_band.p;
   tp->maskf = c->d_tp_maskf.p;
   tp->nrad = c->d_tp_int.p;
   tp->nazm = c->d_tp_int.p + nt;
+  tp->nband = c->d_tp_int.p + 2 * nt;
   return RBC3D_OK;
 }
 
@@ -2599,6 +2745,7 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   int nb = c->nfbins;
   TypePtrs tpv, *tp = &tpv;
   RBC_TRY(rbc_type_ptrs(c, tp));
+  const bool own = cacheable;  // the targets are the cells' own nodes, in order
   cacheable = cacheable && c->geom_reuse;
   const bool hit = cacheable && c->cache_epoch == c->geom_epoch && c->cache_nT == nT;
   c->cache_epoch = -1;  // valid again only when this call completes as cacheable
@@ -2817,7 +2964,32 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   sa.work_cnt = c->d_work_cnt.p;
   sa.dvitem = c->d_dvitem.p;
   rbc_stage_begin(c, ST_SELF);
-  k_self<<<(unsigned)(((size_t)nT * 64 + 255) / 256), 256, 0, st>>>(sa);
+  // by latitude rows where they fill half the compute units or more (one workgroup a unit:
+  // 208 rows of 13 x 26 cells 38 us against 53, 104 rows 35 against 31)
+  if (own && c1 == 0 && c->self_lds > 0 && 2 * c->self_nrow >= c->ncu) {
+    SelfArgs se;
+    se.nT = nT;
+    se.rc = c->conf.rc;
+    se.reps = c->r_eps;
+    se.c2 = c2;
+    se.cells = c->d_cells.p;
+    se.rowlist = (const int2 *)c->d_self_rows.p;
+    se.spl = c->d_spl.p;
+    se.dl1 = c->d_dl1.p;
+    se.th = tp->th;
+    se.phi = tp->phi;
+    se.thG = tp->thG;
+    se.phiS = tp->phiS;
+    se.pwt = tp->pwt;
+    se.rows = tp->band;
+    se.nrad = tp->nrad;
+    se.nazm = tp->nazm;
+    se.nband = tp->nband;
+    se.dvself = dvself;
+    k_self_own<<<c->self_nrow, SELF_T, c->self_lds, st>>>(se);
+  } else {
+    k_self<<<(unsigned)(((size_t)nT * 64 + 255) / 256), 256, 0, st>>>(sa);
+  }
   rbc_stage_end(c, ST_SELF);
   HIP_TRY(hipGetLastError());
   if (nitems > 0 && hit) {
