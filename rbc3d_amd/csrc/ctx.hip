@@ -215,7 +215,14 @@ static int make_gtype(rbc3d_ctx *c, int nlat, GridType **out) {
       }
     return D;
   };
-  RBC_TRY(upload(g->d_Dm, dmat(2 * nl), st));
+  {
+    // (transposed: the threads of a row read consecutive p)
+    const std::vector<double> D = dmat(2 * nl);
+    std::vector<double> Dt(D.size());
+    for (int p = 0; p < 2 * nl; p++)
+      for (int q = 0; q < 2 * nl; q++) Dt[p + (size_t)2 * nl * q] = D[(size_t)2 * nl * p + q];
+    RBC_TRY(upload(g->d_Dm, Dt, st));
+  }
   RBC_TRY(upload(g->d_Dn, dmat(nn), st));
   // polar patch (RbcPolarPatch_Create, common/ModPolarPatch.F90:27-75)
   std::vector<double> mt(RBC_NTAB + 1);

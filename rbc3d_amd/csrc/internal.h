@@ -82,7 +82,7 @@ struct GridType {
   DBuf<double> d_pg;     // synthesis [m][n][i] = Pbar(m,n,th_i) (x 1/2 for m = 0)
   DBuf<double> d_pe;     // equi synthesis, nlat+1 rows incl. poles, [m][n][ie]
   DBuf<double> d_cs;     // cos(m phi_j) [m][j] then sin(m phi_j) [m][j], m <= nlat
-  DBuf<double> d_Dm;     // periodic derivative matrix, length 2 nlat, [p][q]
+  DBuf<double> d_Dm;     // periodic derivative matrix, length 2 nlat, [q][p]
   DBuf<double> d_Dn;     // periodic derivative matrix, length nlon, [p][q]
   DBuf<double> d_thG, d_phiG, d_pwt;  // polar patch: [node][irad + nrad*iazm], weights
   // the patches of one latitude row: longitudes [ilat][point][ilon], and the band of nband

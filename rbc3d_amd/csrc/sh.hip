@@ -27,17 +27,21 @@ struct SplTabs {
   const double *pw[SH_MAXSEG], *pe[SH_MAXSEG], *cs[SH_MAXSEG], *Dm[SH_MAXSEG], *Dn[SH_MAXSEG];
 };
 
-// One persistent launch over the cells of every grid type: each workgroup takes cells
-// in turn (cells of different sizes side by side) with its type's tables.
+// One persistent launch over the cells of every grid type: each workgroup takes one
+// variable of a cell at a time (cells of different sizes side by side) with its type's
+// tables.  A variable is a chain of small contractions that a workgroup's few wavefronts
+// wait for, so a few cells fill the chip better by variables than by cells (24 cells of
+// 13 x 26: 77 -> 36 us).
 __global__ void __launch_bounds__(SH_THREADS) k_build_splines(
     const CellRec *__restrict__ cells, int cell0, SplTabs T, const double *__restrict__ x,
     const double *__restrict__ a3, const double *__restrict__ detj, const double *__restrict__ fd,
     int np, int which, double *__restrict__ spl, const int *__restrict__ cell_list) {
 #pragma clang fp contract(off)
   extern __shared__ double sm[];
-  for (int w = blockIdx.x; w < T.ncell; w += gridDim.x) {
-  __syncthreads();  // the previous cell is done with the LDS buffers
-  int ci = cell_list[cell0 + w];
+  const int nvar = which == 0 ? 7 : 3;
+  for (int w = blockIdx.x; w < T.ncell * nvar; w += gridDim.x) {
+  __syncthreads();  // the previous one is done with the LDS buffers
+  const int v = w % nvar, ci = cell_list[cell0 + w / nvar];
   const CellRec cr = cells[ci];
   int k = 0;
   while (k < SH_MAXSEG - 1 && T.gt[k] != cr.gtype) k++;
@@ -46,8 +50,7 @@ __global__ void __launch_bounds__(SH_THREADS) k_build_splines(
   int mmax = min(nl, nn / 2 + 1);
   int R1 = ne * nn, R2 = 2 * ne * nl;
   double *r1 = sm, *r2 = sm + R1, *u = r2 + R2, *u1 = u + m2 * nn;
-  int nvar = which == 0 ? 7 : 3;
-  for (int v = 0; v < nvar; v++) {
+  {
     // field values on the Gauss grid
     const double *src;
     int comp, var;
@@ -100,7 +103,7 @@ __global__ void __launch_bounds__(SH_THREADS) k_build_splines(
     for (int t = threadIdx.x; t < m2 * nn; t += blockDim.x) {
       int i = t % m2, j = t / m2;
       double s = 0;
-      for (int q = 0; q < m2; q++) s += Dm[i * m2 + q] * u[q + m2 * j];
+      for (int q = 0; q < m2; q++) s += Dm[i + m2 * q] * u[q + m2 * j];
       u1[t] = s;
     }
     __syncthreads();
@@ -190,7 +193,7 @@ int rbc_sh_build_splines(rbc3d_ctx *c, int which) {
     for (int k = nseg; k < SH_MAXSEG; k++) T.gt[k] = -1;
     T.ncell = ncell;
     rbc_stage_begin(c, ST_SPLINE);
-    hipLaunchKernelGGL(k_build_splines, dim3(persistent_grid(c, ncell, 4)), dim3(SH_THREADS), lds,
+    hipLaunchKernelGGL(k_build_splines, dim3(persistent_grid(c, ncell * (which == 0 ? 7 : 3), 4)), dim3(SH_THREADS), lds,
                        c->stream, c->d_cells.p, base, T, c->d_x.p, c->d_a3.p, c->d_detj.p, fd, c->np,
                        which, c->d_spl.p, c->d_tmp_i.p);
     rbc_stage_end(c, ST_SPLINE);
