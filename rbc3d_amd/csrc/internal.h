@@ -294,7 +294,7 @@ struct rbc3d_ctx {
   unsigned long long last_checksum = 0;
   // the PME spread's sort of the cell sources by brick depends on the geometry only:
   // kept for the geometry epoch it was made at (with geometry reuse on)
-  int spread_sort_epoch = -1, spread_sort_ns = 0;
+  int spread_sort_epoch = -1, spread_sort_ns = 0, spread_sort_edge = 0;
   // hipGraph of the cell matvec at fixed geometry (rbc3d_set_graph): captured on the
   // matvec's own input and output buffers, valid for one geometry epoch, precision
   // form and buffer-allocation count
@@ -337,6 +337,13 @@ struct rbc3d_ctx {
   DBuf<double> d_rep_sph, d_rep_dx, d_rep_stat;
   DBuf<int> d_rep_cnt, d_rep_cand_c, d_rep_cand_e;
 };
+
+// whether any cell carries a double layer (Bcoef = 1 - viscosity ratio is not zero)
+inline bool rbc_any_double_layer(const rbc3d_ctx *c) {
+  for (const CellRec &r : c->cells)
+    if (r.Bcoef != 0.) return true;
+  return false;
+}
 
 // ---------------------------------------------------------------------------
 // Device helpers shared by several kernels.

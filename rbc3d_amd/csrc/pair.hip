@@ -2840,9 +2840,7 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
     const unsigned grid = (unsigned)std::min<size_t>(c->ncu, ncl_max);
     // cells of viscosity ratio 1 have no double layer (its density carries Bcoef = 0); the
     // reciprocal part still takes it, so an undefined density shows in every velocity
-    bool dl = false;
-    for (const CellRec &r : c->cells) dl = dl || r.Bcoef != 0.;
-    dl = dl && c2 != 0;
+    const bool dl = c2 != 0 && rbc_any_double_layer(c);
     if (c1 != 0 && dl)
       k_pair<true, true><<<grid, 64 * 12, 0, st>>>(pa);
     else if (c1 != 0)
