@@ -586,8 +586,8 @@ extern "C" int rbc3d_destroy(rbc3d_ctx *c) {
   }
   for (DBuf<double> *b : {&c->d_sl1, &c->d_sl2, &c->d_dl1, &c->d_mtab, &c->d_x, &c->d_a3, &c->d_detj,
                           &c->d_ds, &c->d_f, &c->d_g, &c->d_fs, &c->d_gs, &c->d_spl, &c->d_src_rec,
-                          &c->d_tx, &c->d_tA, &c->d_v, &c->d_vacc, &c->d_nbr_dist, &c->d_dvitem,
-                          &c->d_scratch, &c->d_cell_sph, &c->d_chunk_sph, &c->d_grid, &c->d_cgrid, &c->d_vgrid,
+                          &c->d_tx, &c->d_tA, &c->d_v, &c->d_vacc, &c->d_dvitem,
+                          &c->d_scratch, &c->d_cell_sph, &c->d_grid, &c->d_cgrid, &c->d_vgrid,
                           &c->d_bb, &c->d_tw, &c->d_pme_src, &c->d_shbuf, &c->d_shbuf2,
                           &c->wall.d_x, &c->wall.d_f, &c->wall.d_area, &c->wall.d_eps,
                           &c->wall.d_cen, &c->wall.d_val})
@@ -635,7 +635,7 @@ extern "C" int rbc3d_set_cells(rbc3d_ctx *c, int nrbc, const int *nlat0, const i
   const int prev_nrbc = c->nrbc;
   c->nrbc = nrbc;
   c->cells.resize(nrbc);
-  int np = 0, coff = 0, choff = 0;
+  int np = 0, coff = 0;
   long long spl = 0;
   for (int i = 0; i < nrbc; i++) {
     if (nlat[i] < 2 || nlat[i] > 64 || nlat0[i] < 1 || nlat0[i] > nlat[i] || celltype[i] < 1 ||
@@ -658,8 +658,6 @@ extern "C" int rbc3d_set_cells(rbc3d_ctx *c, int nrbc, const int *nlat0, const i
     r.spl = spl;
     r.coff = coff;
     coff += 3 * r.nlat0 * r.nlat0;
-    r.choff = choff;
-    choff += (r.nlat * r.nlon + 63) / 64;
     int npt = g->nlat * g->nlon;
     // area and mesh size (RBC_ComputeGeometry, common/ModRbc.F90:482-505)
     double area = 0;
@@ -674,7 +672,6 @@ extern "C" int rbc3d_set_cells(rbc3d_ctx *c, int nrbc, const int *nlat0, const i
   c->np = np;
   c->sbq_ready = false;
   c->x_moved = false;
-  c->nchunks = choff;
   c->geom_epoch++;
   // the previous cell-BIE solution is the next solve's initial guess only for the same
   // set of unknowns

@@ -139,7 +139,6 @@ struct CellRec {
   int nlat, nlon, nlat0;
   int celltype;  // 1-based
   int coff;      // offset of the cell's block in the Glob_Sph_Trans vector
-  int choff;     // first 64-node chunk of the cell (chunk bounding spheres)
   long long spl;  // offset (doubles) of the cell's spline block
   double Acoef, Bcoef, area, meshSize, radius;
 };
@@ -235,17 +234,15 @@ struct rbc3d_ctx {
   DBuf<int> d_clus;  // the pair kernel's target clusters: (fine bin, first sorted target)
   DBuf<int> d_nbr_cnt, d_nbr_cell, d_nbr_node;
   DBuf<int> d_cell_cand;  // per cell: candidate neighbouring cells, then their counts
-  DBuf<double> d_nbr_dist;
   DBuf<int> d_work, d_work_cnt;
   DBuf<double> d_dvitem, d_scratch;
   DBuf<int> d_flag;
   DBuf<unsigned long long> d_pairstat;
   // cell bounding spheres binned by centre (neighbour-cell candidates)
   DBuf<double> d_cell_sph;
-  DBuf<double> d_chunk_sph;  // per 64-node chunk of every cell: centre(3), radius
+  DBuf<float> d_nodeoff;     // nodes relative to their cell's centre, FP32 [d][np]
   DBuf<int> d_src_cc;        // coarse cell-list coordinates per node (packed)
   DBuf<double> d_shx;        // SH Legendre GEMM operands (m, row, col) x 2
-  int nchunks = 0;
   DBuf<int> d_cellbin_start, d_cellbin_order;
   double max_cell_radius = 0;
   // PME

@@ -379,9 +379,10 @@ __global__ void k_density(int np, const double *__restrict__ src, const double *
   for (int d = 0; d < 3; d++) dst[p + (size_t)np * d] = src[p + (size_t)np * d] * s;
 }
 
-// bounding sphere of each cell (centroid of nodes, max node distance)
+// bounding sphere of each cell (centroid of nodes, max node distance), and the nodes
+// relative to its centre in FP32 (k_nbr's sweep)
 __global__ void k_cell_sphere(int nrbc, const CellRec *__restrict__ cells, const double *__restrict__ x,
-                              int np, double *sph) {
+                              int np, double *sph, float *xo) {
   int ci = blockIdx.x;
   if (ci >= nrbc) return;
   const CellRec cr = cells[ci];
@@ -405,6 +406,7 @@ __global__ void k_cell_sphere(int nrbc, const CellRec *__restrict__ cells, const
     for (int d = 0; d < 3; d++) {
       double dd = x[cr.off + t + (size_t)np * d] - cen[d];
       r2 += dd * dd;
+      xo[cr.off + t + (size_t)np * d] = (float)dd;
     }
     rmax = fmax(rmax, sqrt(r2));
   }
@@ -419,39 +421,6 @@ __global__ void k_cell_sphere(int nrbc, const CellRec *__restrict__ cells, const
     sph[4 * ci + 1] = cen[1];
     sph[4 * ci + 2] = cen[2];
     sph[4 * ci + 3] = red[3][0] * (1 + 1e-12) + 1e-12;
-  }
-}
-
-// bounding spheres of each cell's consecutive 64-node chunks: one wavefront per chunk
-__global__ void k_chunk_sphere(int nrbc, const CellRec *__restrict__ cells,
-                               const double *__restrict__ x, int np, double *sph) {
-  const int ci = blockIdx.x;
-  if (ci >= nrbc) return;
-  const CellRec cr = cells[ci];
-  const int npt = cr.nlat * cr.nlon, nch = (npt + 63) / 64;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int k = wv; k < nch; k += nw) {
-    const int q = 64 * k + lane, cnt = min(64, npt - 64 * k);
-    double p[3] = {0, 0, 0};
-    if (q < npt)
-      for (int d = 0; d < 3; d++) p[d] = x[cr.off + q + (size_t)np * d];
-    double cen[3];
-    for (int d = 0; d < 3; d++) {
-      double v = p[d];
-      for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-      cen[d] = v / cnt;
-    }
-    double r2 = 0;
-    if (q < npt)
-      for (int d = 0; d < 3; d++) r2 += (p[d] - cen[d]) * (p[d] - cen[d]);
-    for (int o = 32; o > 0; o >>= 1) r2 = fmax(r2, __shfl_xor(r2, o, 64));
-    if (lane == 0) {
-      double *s = sph + 4 * (size_t)(cr.choff + k);
-      s[0] = cen[0];
-      s[1] = cen[1];
-      s[2] = cen[2];
-      s[3] = sqrt(r2) * (1 + 1e-12) + 1e-12;
-    }
   }
 }
 
@@ -499,7 +468,9 @@ int rbc_build_source_list(rbc3d_ctx *c) {
   RBC_TRY(fine_sort(c, np, c->d_x.p, np, c->d_tmp_f.p, c->d_src_order.p, c->d_fbin_start.p));
   RBC_TRY(c->d_src_rec.ensure((size_t)SREC * np + 1));
   RBC_TRY(c->d_cell_sph.ensure((size_t)4 * c->nrbc + 4));
-  k_cell_sphere<<<c->nrbc, 256, 0, c->stream>>>(c->nrbc, c->d_cells.p, c->d_x.p, np, c->d_cell_sph.p);
+  RBC_TRY(c->d_nodeoff.ensure((size_t)3 * np + 1));
+  k_cell_sphere<<<c->nrbc, 256, 0, c->stream>>>(c->nrbc, c->d_cells.p, c->d_x.p, np, c->d_cell_sph.p,
+                                                c->d_nodeoff.p);
   HIP_TRY(hipGetLastError());
   RBC_TRY(c->d_src_cc.ensure(np + 1));
   {
@@ -511,9 +482,6 @@ int rbc_build_source_list(rbc3d_ctx *c) {
     k_coarse_coords<<<(np + 255) / 256, 256, 0, c->stream>>>(np, c->d_x.p, hg, c->d_src_cc.p);
     HIP_TRY(hipGetLastError());
   }
-  RBC_TRY(c->d_chunk_sph.ensure((size_t)4 * c->nchunks + 4));
-  k_chunk_sphere<<<c->nrbc, 256, 0, c->stream>>>(c->nrbc, c->d_cells.p, c->d_x.p, np,
-                                                 c->d_chunk_sph.p);
   HIP_TRY(hipGetLastError());
   return rbc_update_density(c, 0);
 }
@@ -1808,21 +1776,20 @@ __global__ void __launch_bounds__(PT *PW) k_pair32(Pair32Args a) {
 // neighbouring-cell lists: for every target and every other cell with a node in the
 // cut-off, the closest node (ties: first visited, i.e. lowest 27-bin visit position
 // of the reference's cell list, then highest source index), NbrRbcList_Insert.
-// One wavefront per target: lanes test the cells' bounding spheres, then sweep the
-// nodes of each candidate cell and reduce (distance, visit key, node).
 struct NbrArgs {
   double Lb[3], iLb[3], iLbNc[3];
+  float fLb[3], fiLb[3], fLmin, fLmax;
   int Nc[3];
   double rc;
   int np, nT, nrbc;
   const double *x;  // node coordinates [d][np]
   const int *src_cc;  // coarse bin coordinates per node, packed 10 bits each
   const CellRec *cells;
-  const double *sph, *chunk_sph;
+  const double *sph;
+  const float *xo;  // nodes relative to their cell's centre, FP32 [d][np]
   const double *tx;
   const int *tindx, *tact;
   int *cnt, *slot_cell, *slot_node;
-  double *slot_dist;
   int *flag;
   const int *cand, *ccnt;  // per cell: cells within reach of any of its nodes (k_cell_cands)
 };
@@ -1867,13 +1834,61 @@ __device__ __forceinline__ bool nbr_better(double r1, int k1, int n1, double r2,
   return n1 > n2;
 }
 
-// One wavefront per target: lanes test the cells' bounding spheres; for each cell
-// that passes they test its 64-node chunk spheres and sweep the nodes of the chunks
-// that reach within rc, then reduce (distance, visit key, node) over the wavefront.
-// Cells enter the list in increasing index order.
+// minimum over the wavefront, in every lane's scalar copy: DPP steps within rows of 16
+// lanes, then the rows' results passed on to lane 63
+__device__ __forceinline__ float wave_min_f(float v) {
+#define NBR_DPP(ctrl, rmask) \
+  v = fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), \
+                                                          ctrl, rmask, 0xf, false)))
+  NBR_DPP(0xB1, 0xf);   // quad_perm(1,0,3,2)
+  NBR_DPP(0x4E, 0xf);   // quad_perm(2,3,0,1)
+  NBR_DPP(0x141, 0xf);  // row_half_mirror
+  NBR_DPP(0x140, 0xf);  // row_mirror
+  NBR_DPP(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+  NBR_DPP(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef NBR_DPP
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// squared FP32 distances of one cell's nodes (64 a step, the last node repeated past the
+// end) from the target at t relative to the cell's centre: the lane's two smallest and the
+// first's byte offset.  Byte offsets in 32 bits keep the addresses to one register.
+template <bool WRAP>
+__device__ __forceinline__ void nbr_sweep(const NbrArgs &a, const char *x0, const char *x1,
+                                          const char *x2, int npt, int lane, const float t[3],
+                                          float &b1, float &b2, unsigned &bo) {
+  const unsigned end = 4u * (unsigned)(npt - 1);
+  const int nch = (npt + 63) >> 6;
+  unsigned o = 4u * lane;
+#pragma unroll 4
+  for (int k = 0; k < nch; k++, o += 256) {
+    const unsigned q = min(o, end);
+    float d0 = *(const float *)(x0 + q) - t[0], d1 = *(const float *)(x1 + q) - t[1],
+          d2 = *(const float *)(x2 + q) - t[2];
+    if (WRAP) {
+      d0 -= rintf(d0 * a.fiLb[0]) * a.fLb[0];
+      d1 -= rintf(d1 * a.fiLb[1]) * a.fLb[1];
+      d2 -= rintf(d2 * a.fiLb[2]) * a.fLb[2];
+    }
+    const float r2 = fmaf(d2, d2, fmaf(d1, d1, d0 * d0));
+    b2 = __builtin_amdgcn_fmed3f(b1, b2, r2);  // b1 <= b2
+    bo = r2 < b1 ? q : bo;
+    b1 = r2 < b1 ? r2 : b1;
+  }
+}
+
+// One wavefront per target: lanes test the cells' bounding spheres; for each cell that
+// passes they sweep its nodes in FP32 relative to the cell's centre, and only the nodes
+// within twice the sweep's error bound of its smallest distance (nearly always one) are
+// evaluated in FP64, reduced by (distance, visit key, node).  Cells enter the list in
+// increasing index order.
+// What bounds it: VALU issue (about 15 cells within reach of a target), with the loads of
+// the sweep close behind.  The FP64 sweep behind bounding spheres of 64-node strips that
+// was here took some 600 instructions a cell.  296k targets on 512 cells 4.54 -> 1.33
+// ms; on 4096 cells of mixed grids 17.0 -> 5.4 ms; 20,000 points among 128 cells 353 -> 104 us.
 __global__ void __launch_bounds__(NBR_T) k_nbr(NbrArgs a) {
   const int lane = threadIdx.x & 63;
-  const int ti = (blockIdx.x * NBR_T + (int)threadIdx.x) >> 6;
+  const int ti = __builtin_amdgcn_readfirstlane((blockIdx.x * NBR_T + (int)threadIdx.x) >> 6);
   if (ti >= a.nT) return;
   if (!a.tact[ti]) {
     if (lane == 0) a.cnt[ti] = 0;
@@ -1889,6 +1904,7 @@ __global__ void __launch_bounds__(NBR_T) k_nbr(NbrArgs a) {
   int n = 0;
   bool ovf = false;
   const size_t np = a.np;
+  const float frc = (float)a.rc;
   // the cells to test: the candidate list of the target's own cell when the target
   // lies within that cell's bounding sphere, else every cell
   const int *clist = nullptr;
@@ -1906,36 +1922,72 @@ __global__ void __launch_bounds__(NBR_T) k_nbr(NbrArgs a) {
     const int idx = cbase + lane;
     const int cj = idx < ncl ? (clist ? clist[idx] : idx) : -1;
     bool pass = false;
+    float tc0 = 0, tc1 = 0, tc2 = 0, trad = 0;
+    int toff = 0, tnpt = 0;
     if (cj >= 0 && cj != surf_i - 1) {
       double cen[3] = {a.sph[4 * cj], a.sph[4 * cj + 1], a.sph[4 * cj + 2]}, dd[3];
       double rcen = ref_min_image_dist(xi, cen, a.Lb, a.iLb, dd);
       pass = !(rcen > a.rc + a.sph[4 * cj + 3] + 1e-9 * a.rc);
+      tc0 = -(float)dd[0];
+      tc1 = -(float)dd[1];
+      tc2 = -(float)dd[2];
+      trad = (float)a.sph[4 * cj + 3];
+      toff = a.cells[cj].off;
+      tnpt = a.cells[cj].nlat * a.cells[cj].nlon;
     }
     unsigned long long m = __ballot(pass);
     while (m) {
-      int kk = __ffsll((long long)m) - 1;
+      const int kk = __ffsll((long long)m) - 1;
       m &= m - 1;
-      int c2 = __shfl(cj, kk, 64);
-      const CellRec cr = a.cells[c2];
-      int npt = cr.nlat * cr.nlon, nch = (npt + 63) / 64;
+      const int c2 = __builtin_amdgcn_readlane(cj, kk);
+      auto lane_f = [kk](float v) {
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), kk));
+      };
+      const float t[3] = {lane_f(tc0), lane_f(tc1), lane_f(tc2)}, sr = lane_f(trad);
+      const int off = __builtin_amdgcn_readlane(toff, kk), npt = __builtin_amdgcn_readlane(tnpt, kk);
+      const float *x0 = a.xo + off, *x1 = x0 + np, *x2 = x1 + np;
+      // error of a squared FP32 distance: coordinates, their differences and (in a box
+      // that the cell's far nodes wrap around) the box length are rounded at 2^-24 of at
+      // most M, three or four times an axis: below 24 * 2^-24 M^2
+      const bool wrap = !(a.fLmin > 2.001f * (frc + sr));
+      const float M = frc + 2 * sr + (wrap ? a.fLmax : 0.f), tol = M * M * 3.8e-6f;
+      float b1 = 3e38f, b2 = 3e38f;
+      unsigned bo = 0;
+      if (wrap)
+        nbr_sweep<true>(a, (const char *)x0, (const char *)x1, (const char *)x2, npt, lane, t, b1, b2, bo);
+      else
+        nbr_sweep<false>(a, (const char *)x0, (const char *)x1, (const char *)x2, npt, lane, t, b1, b2, bo);
+      const int bq = (int)(bo >> 2);
+      const float bm = wave_min_f(b1);
+      // no node within rc; a target or cell that is not a number takes the full sweep
+      const bool nan = !(t[0] + t[1] + t[2] + sr < 3e38f);
+      if (!nan && bm > frc * frc * (1 + 1e-6f) + tol) continue;
+      float lim = nan ? __builtin_inff() : bm + 2 * tol;
+      bool all = nan || __ballot(b2 <= lim) != 0ull;  // a lane holds several candidates
+      const unsigned long long cm = __ballot(b1 <= lim);
+      if (!all && (cm & (cm - 1)) == 0ull && bm < frc * frc * (1 - 1e-6f) - tol && n < RBC_NBR_MAX) {
+        // one candidate, surely within rc and so, by far more than the rounding of the bin
+        // coordinates, within the 27 bins (no narrower than rc)
+        if (b1 <= lim) {
+          const size_t s = (size_t)ti * RBC_NBR_MAX + n;
+          a.slot_cell[s] = c2;
+          a.slot_node[s] = off + bq;
+        }
+        n++;
+        continue;
+      }
       double best = 0;
       int bkey = 0, bnode = -1;
-      // only the 64-node chunks whose bounding sphere reaches within rc of the target
-      for (int cb = 0; cb < nch; cb += 64) {
-        bool cp = false;
-        if (cb + lane < nch) {
-          const double *s = a.chunk_sph + 4 * (size_t)(cr.choff + cb + lane);
-          double cen[3] = {s[0], s[1], s[2]}, dd[3];
-          double rcen = ref_min_image_dist(xi, cen, a.Lb, a.iLb, dd);
-          cp = !(rcen > a.rc + s[3] + 1e-9 * a.rc);
-        }
-        unsigned long long cm = __ballot(cp);
-        while (cm) {
-          const int kc = cb + __ffsll((long long)cm) - 1;
-          cm &= cm - 1;
-          const int q = 64 * kc + lane;
-          if (q >= npt) continue;
-          const int node = cr.off + q;
+      while (true) {
+        bool outside = false;  // a candidate within rc that the 27 bins leave out
+        for (int q = all ? lane : bq; q < npt; q += all ? 64 : npt) {
+          if (!nan) {
+            float d[3] = {x0[q] - t[0], x1[q] - t[1], x2[q] - t[2]};
+            for (int k = 0; k < 3; k++)
+              if (wrap) d[k] -= rintf(d[k] * a.fiLb[k]) * a.fLb[k];
+            if (fmaf(d[2], d[2], fmaf(d[1], d[1], d[0] * d[0])) > lim) continue;
+          }
+          const int node = off + q;
           double xj[3] = {a.x[node], a.x[node + np], a.x[node + 2 * np]}, xx[3];
           double rr = ref_min_image_dist(xi, xj, a.Lb, a.iLb, xx);
           if (rr > a.rc) continue;
@@ -1944,7 +1996,10 @@ __global__ void __launch_bounds__(NBR_T) k_nbr(NbrArgs a) {
           d1 += d1 < 0 ? a.Nc[0] : (d1 >= a.Nc[0] ? -a.Nc[0] : 0);
           d2 += d2 < 0 ? a.Nc[1] : (d2 >= a.Nc[1] ? -a.Nc[1] : 0);
           d3 += d3 < 0 ? a.Nc[2] : (d3 >= a.Nc[2] ? -a.Nc[2] : 0);
-          if (d1 > 2 || d2 > 2 || d3 > 2) continue;  // not in the 27 visited bins
+          if (d1 > 2 || d2 > 2 || d3 > 2) {  // not in the 27 visited bins
+            outside = true;
+            continue;
+          }
           const int key = 9 * d1 + 3 * d2 + d3;
           if (nbr_better(rr, key, node, best, bkey, bnode)) {
             best = rr;
@@ -1952,29 +2007,31 @@ __global__ void __launch_bounds__(NBR_T) k_nbr(NbrArgs a) {
             bnode = node;
           }
         }
+        if (__ballot(bnode >= 0) != 0ull || __ballot(outside) == 0ull || lim >= 3e38f) break;
+        lim = 3.2e38f;  // every candidate was left out: look at all nodes
+        all = true;
       }
-      if (__ballot(bnode >= 0) == 0ull) continue;  // no node of this cell within rc
-      for (int o = 32; o > 0; o >>= 1) {
-        double ob = __shfl_xor(best, o, 64);
-        int ok = __shfl_xor(bkey, o, 64), on = __shfl_xor(bnode, o, 64);
-        if (nbr_better(ob, ok, on, best, bkey, bnode)) {
-          best = ob;
-          bkey = ok;
-          bnode = on;
-        }
-      }
-      if (bnode >= 0) {
-        if (n < RBC_NBR_MAX) {
-          if (lane == 0) {
-            size_t s = (size_t)ti * RBC_NBR_MAX + n;
-            a.slot_cell[s] = c2;
-            a.slot_node[s] = bnode;
-            a.slot_dist[s] = best;
+      const unsigned long long found = __ballot(bnode >= 0);
+      if (found == 0ull) continue;  // no node of this cell within rc
+      if (found & (found - 1))
+        for (int o = 32; o > 0; o >>= 1) {
+          double ob = __shfl_xor(best, o, 64);
+          int ok = __shfl_xor(bkey, o, 64), on = __shfl_xor(bnode, o, 64);
+          if (nbr_better(ob, ok, on, best, bkey, bnode)) {
+            best = ob;
+            bkey = ok;
+            bnode = on;
           }
-          n++;
-        } else {
-          ovf = true;
         }
+      if (n < RBC_NBR_MAX) {
+        if (lane == __ffsll((long long)found) - 1) {
+          const size_t s = (size_t)ti * RBC_NBR_MAX + n;
+          a.slot_cell[s] = c2;
+          a.slot_node[s] = bnode;
+        }
+        n++;
+      } else {
+        ovf = true;
       }
     }
   }
@@ -2858,14 +2915,17 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   RBC_TRY(c->d_nbr_cnt.ensure(2 * (size_t)nT + 2));
   RBC_TRY(c->d_nbr_cell.ensure((size_t)RBC_NBR_MAX * nT + 1));
   RBC_TRY(c->d_nbr_node.ensure((size_t)RBC_NBR_MAX * nT + 1));
-  RBC_TRY(c->d_nbr_dist.ensure((size_t)RBC_NBR_MAX * nT + 1));
   NbrArgs na;
   for (int d = 0; d < 3; d++) {
     na.Lb[d] = c->Lb[d];
     na.iLb[d] = c->iLb[d];
     na.iLbNc[d] = c->iLbNc[d];
     na.Nc[d] = c->Nc[d];
+    na.fLb[d] = (float)c->Lb[d];
+    na.fiLb[d] = (float)c->iLb[d];
   }
+  na.fLmin = std::min(na.fLb[0], std::min(na.fLb[1], na.fLb[2]));
+  na.fLmax = std::max(na.fLb[0], std::max(na.fLb[1], na.fLb[2]));
   na.rc = c->conf.rc;
   na.np = c->np;
   na.nT = nT;
@@ -2874,14 +2934,13 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   na.src_cc = c->d_src_cc.p;
   na.cells = c->d_cells.p;
   na.sph = c->d_cell_sph.p;
-  na.chunk_sph = c->d_chunk_sph.p;
+  na.xo = c->d_nodeoff.p;
   na.tx = d_tx;
   na.tindx = d_tindx;
   na.tact = d_act;
   na.cnt = c->d_nbr_cnt.p;
   na.slot_cell = c->d_nbr_cell.p;
   na.slot_node = c->d_nbr_node.p;
-  na.slot_dist = c->d_nbr_dist.p;
   na.flag = c->d_flag.p;
   RBC_TRY(c->d_cell_cand.ensure((size_t)(RBC_CAND_MAX + 1) * c->nrbc + 1));
   na.cand = c->d_cell_cand.p;
