@@ -19,11 +19,17 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-result"]
+# The FP64 constants of the sines, arc cosines and logarithms are hoisted out of the
+# near-singular kernels' loops into some hundred registers by machine-level LICM, which then
+# run at 2 wavefronts a SIMD or spill.  Left in place they are scalar moves beside the vector
+# work: the projection 3.41 -> 3.13 ms, the correction 0.97 -> 0.79 ms (512 cells of 17 x 34
+# nodes); the file's other kernels are unchanged.
+FILE_FLAGS = {"pair.hip": ["-mllvm", "-disable-machine-licm"]}
 
 
 def _compile(src):
     obj = os.path.join(OBJ, src.replace(".hip", ".o"))
-    cmd = [HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [HIPCC, *FLAGS, *FILE_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr[-4000:]}")

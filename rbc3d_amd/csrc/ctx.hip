@@ -475,6 +475,7 @@ extern "C" int rbc3d_create(const rbc3d_conf *conf, rbc3d_ctx **out) {
   if (!r) r = upload(c->d_sl2, t2, c->stream);
   if (!r) r = upload(c->d_dl1, t3, c->stream);
   if (!r) r = upload(c->d_mtab, mt, c->stream);
+  if (!r) r = rbc_gauleg16(c);
   {
     // the same tables in FP32 for the split form's pair kernel
     std::vector<float> tf(3 * (size_t)(RBC_NTAB + 1));

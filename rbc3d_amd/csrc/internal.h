@@ -200,6 +200,7 @@ struct rbc3d_ctx {
   int lds_max = 65536;         // LDS bytes one workgroup may allocate on the device
   // tables
   DBuf<double> d_sl1, d_sl2, d_dl1, d_mtab;
+  DBuf<double> d_gl16;  // roots and derivatives of GauLeg with 16 nodes (k_gauleg16)
   DBuf<float> d_tabf;  // split form: sl1, sl2, dl1 in FP32, (RBC_NTAB + 1) each
   double r_eps;
   // cell list geometry
@@ -566,6 +567,7 @@ int rbc_sh_anal_batch(int nlat, int nlon, int nt, const double *d_g, int idg, in
 int rbc_sh_synth_batch(int nlat, int nlon, int nt, double *d_g, int idg, int jdg, const double *d_a,
                        const double *d_b, int ida, int jda, int equi, hipStream_t st);
 int rbc_build_source_list(rbc3d_ctx *c);
+int rbc_gauleg16(rbc3d_ctx *c);  // fills d_gl16 (pair.hip)
 int rbc_self_rows(rbc3d_ctx *c);  // launch list of the self patches by latitude rows
 // device arrays of per-grid-type table pointers, indexed by CellRec::gtype (pair.hip):
 // same-surface mask, grid colatitudes and longitudes, patch points and weights, projection

@@ -2068,12 +2068,14 @@ __device__ __forceinline__ void patch_point(double s0, double c0, double phi0, d
   patch_point_sc(s0, c0, phi0, sin(thL), cos(thL), sin(phL), cos(phL), thG, phG);
 }
 
-// GauLeg (common/ModQuadRule.F90:135-208), node k (ascending) and its weight: each root's Newton iteration is
-// independent of the others, so one lane computes one node, as GauLeg does for it.
-__device__ void gauleg_node(double x1, double x2, int n, int k, double &x, double &w) {
-  const int m = (n + 1) / 2;
-  const int j = k < m ? k : n - 1 - k;
-  double xm = 0.5 * (x2 + x1), xl = 0.5 * (x2 - x1);
+// GauLeg (common/ModQuadRule.F90:135-208) with the near-singular patch's 16 radial nodes:
+// the Newton iteration for root j of the Legendre polynomial and its derivative there,
+// which do not depend on the interval; lane j < 8 stores (root, derivative).  Once a
+// context: in every correction's wavefront they were some 2000 of its instructions.
+#define RBC_NEAR_NRAD 16
+__global__ void k_gauleg16(double *tab) {
+  const int n = RBC_NEAR_NRAD, j = threadIdx.x;
+  if (j >= n / 2) return;
   double z = cos(RBC_PI * ((j + 1) - 0.25) / (n + 0.5)), z1, p1 = 0, p2, p3, pp = 0;
   bool unfinished = true;
   for (int its = 1; its <= 10 && unfinished; its++) {
@@ -2089,21 +2091,38 @@ __device__ void gauleg_node(double x1, double x2, int n, int k, double &x, doubl
     z = z1 - p1 / pp;
     unfinished = fabs(z - z1) > 3.e-14;
   }
-  // GauLeg writes x(j) then x(n-1-j); for the middle node of odd n the second wins
+  tab[2 * j] = z;
+  tab[2 * j + 1] = pp;
+}
+
+int rbc_gauleg16(rbc3d_ctx *c) {
+  RBC_TRY(c->d_gl16.ensure(RBC_NEAR_NRAD));
+  k_gauleg16<<<1, 64, 0, c->stream>>>(c->d_gl16.p);
+  HIP_TRY(hipGetLastError());
+  return RBC3D_OK;
+}
+
+// node k (ascending) of GauLeg on [x1, x2] and its weight, from the table of k_gauleg16
+__device__ __forceinline__ void gauleg_node(const double *__restrict__ gl, double x1, double x2,
+                                            int k, double &x, double &w) {
+  const int n = RBC_NEAR_NRAD, j = k < n / 2 ? k : n - 1 - k;
+  const double xm = 0.5 * (x2 + x1), xl = 0.5 * (x2 - x1);
+  const double z = gl[2 * j], pp = gl[2 * j + 1];
   x = (k == n - 1 - j) ? xm + xl * z : xm - xl * z;
   w = 2.0 * xl / ((1.0 - z * z) * pp * pp);
 }
 
 // node k of GauLeg_Sinh (common/ModQuadRule.F90:223-263)
-__device__ void gauleg_sinh_node(double xmin, double xmax, double a, double b, int n, int k,
-                                 double &x, double &w) {
+__device__ __forceinline__ void gauleg_sinh_node(const double *__restrict__ gl, double xmin,
+                                                 double xmax, double a, double b, int k, double &x,
+                                                 double &w) {
   double xm = 0.5 * (xmin + xmax), xl = 0.5 * (xmax - xmin);
   double a0 = (a - xm) / xl, b0 = b * xl;
   double f1 = (1 + a0) / b0, f2 = (1 - a0) / b0;
   double u1 = log(f1 + sqrt(1 + f1 * f1)), u2 = log(f2 + sqrt(1 + f2 * f2));
   double mu = 0.5 * (u1 + u2), eta = 0.5 * (u1 - u2);
   double sk, wk;
-  gauleg_node(-1., 1., n, k, sk, wk);
+  gauleg_node(gl, -1., 1., k, sk, wk);
   double xk = a0 + b0 * sinh(mu * sk - eta);
   wk = wk * b0 * mu * cosh(mu * sk - eta);
   w = xl * wk;
@@ -2118,7 +2137,7 @@ struct SingArgs {
   const double *spl;
   const double *const *th, *const *phi, *const *thG, *const *phiG, *const *pwt;
   const int *nrad, *nazm;
-  const double *sl1, *sl2, *dl1, *mtab;
+  const double *sl1, *sl2, *dl1, *mtab, *gl16;
   const double *x, *fs, *gs, *a3, *detj, *w_unused;
   const double *tx, *tA;
   const int *tindx, *tact;
@@ -2369,7 +2388,128 @@ __global__ void k_items(int nT, const int *__restrict__ cnt, const int *__restri
 }
 
 // RBC_NearSingInt_ReAdd (common/ModRbcSingInt.F90:232-310), lanes over the 16 x 32 patch
-__device__ void readd_wave(const SingArgs &a, const CellRec &cr, const double *blk, int m, int n,
+template <bool SL>
+__device__ __forceinline__ void readd_wave(const SingArgs &a, const CellRec &cr, const double *blk, int m, int n,
+                           const double xi[3], const double x0[3], double th0, double phi0,
+                           double radPat, double c1, double c2, double dv[3]) {
+  const int nrad = RBC_NEAR_NRAD, nazm = 32;
+  // lane l always takes radial node l % 16 (64 is a multiple of nrad): its node and
+  // masked weight are computed once
+  const int lane = threadIdx.x & 63, irad = lane & (nrad - 1);
+  double d0 = xi[0] - x0[0], d1 = xi[1] - x0[1], d2 = xi[2] - x0[2];
+  double dist = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+  double sizePat = radPat * sqrt(cr.area / (4 * RBC_PI));
+  double thl, wl;
+  if (dist > 2.2250738585072014e-308) {
+    dist = dist * (radPat / sizePat);
+    gauleg_sinh_node(a.gl16, 0., radPat, 0., dist, irad, thl, wl);
+  } else {
+    gauleg_node(a.gl16, 0., radPat, irad, thl, wl);
+  }
+  double w = wl * sin(thl) * (RBC_TWO_PI / nazm);
+  w = w * mask_fn(a.mtab, thl / radPat);
+  size_t vs = (size_t)m * n * 4;
+  double s0 = sin(th0), c0 = cos(th0);
+  double a0 = 0, a1 = 0, a2 = 0;
+  // sin and cos of the nazm azimuths, once per wavefront (lane j < nazm: azimuth j, the
+  // same expression as the point loop's), and of the lane's own radial angle
+  __shared__ double azsc[256 / 64][nazm][2];
+  const int wsl = (int)(threadIdx.x >> 6);
+  if (lane < nazm) {
+    const double phL = lane * RBC_TWO_PI / nazm;
+    azsc[wsl][lane][0] = sin(phL);
+    azsc[wsl][lane][1] = cos(phL);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  const double stl = sin(thl), ctl = cos(thl);
+#pragma nounroll
+  for (int p = lane; p < nrad * nazm; p += 64) {
+    int iazm = p / nrad;
+    double thj, phj;
+    patch_point_sc(s0, c0, phi0, stl, ctl, azsc[wsl][iazm][0], azsc[wsl][iazm][1], thj, phj);
+    double xj[3], xx[3];
+    spline_interp(blk + vs * SPL_X, m, n, thj, phj, 3, xj);
+    for (int d = 0; d < 3; d++) xx[d] = xj[d] - xi[d];
+    double rr = sqrt(xx[0] * xx[0] + xx[1] * xx[1] + xx[2] * xx[2]);
+    if (rr > a.rc) continue;
+    if (SL && c1 != 0) {
+      double fj[3], EA, EB;
+      spline_interp(blk + vs * SPL_F, m, n, thj, phj, 3, fj);
+      for (int d = 0; d < 3; d++) fj[d] = w * fj[d];
+      ewald_sl(a.sl1, a.sl2, rr, a.reps, a.rc, EA, EB);
+      double xf = xx[0] * fj[0] + xx[1] * fj[1] + xx[2] * fj[2];
+      a0 += c1 * (EA * xx[0] * xf + EB * fj[0]);
+      a1 += c1 * (EA * xx[1] * xf + EB * fj[1]);
+      a2 += c1 * (EA * xx[2] * xf + EB * fj[2]);
+    }
+    if (c2 != 0) {
+      double gj[3], nj[3];
+      spline_interp(blk + vs * SPL_A3, m, n, thj, phj, 3, nj);
+      spline_interp(blk + vs * SPL_G, m, n, thj, phj, 3, gj);
+      for (int d = 0; d < 3; d++) gj[d] = w * gj[d];
+      double EA = ewald_dl(a.dl1, rr, a.reps, a.rc);
+      double xg = xx[0] * gj[0] + xx[1] * gj[1] + xx[2] * gj[2];
+      double xn = xx[0] * nj[0] + xx[1] * nj[1] + xx[2] * nj[2];
+      a0 += c2 * (EA * xx[0] * xg * xn);
+      a1 += c2 * (EA * xx[1] * xg * xn);
+      a2 += c2 * (EA * xx[2] * xg * xn);
+    }
+  }
+  dv[0] = wave_sum(a0);
+  dv[1] = wave_sum(a1);
+  dv[2] = wave_sum(a2);
+}
+
+// The near-singular correction of calls without a double layer, in the order that it has
+// always summed in: its results enter the walls' velocities, whose solver's iteration count
+// hangs on their last bits (traction to 1e-5), so this path keeps every operation.  The
+// double-layer terms below are never taken here, but without them the compiler contracts
+// the others differently (measured: 3% of the results change in the last bit).
+// GauLeg (common/ModQuadRule.F90:135-208), node k (ascending) and its weight: each root's Newton iteration is
+// independent of the others, so one lane computes one node, as GauLeg does for it.
+__device__ void sl_gauleg_node(double x1, double x2, int n, int k, double &x, double &w) {
+  const int m = (n + 1) / 2;
+  const int j = k < m ? k : n - 1 - k;
+  double xm = 0.5 * (x2 + x1), xl = 0.5 * (x2 - x1);
+  double z = cos(RBC_PI * ((j + 1) - 0.25) / (n + 0.5)), z1, p1 = 0, p2, p3, pp = 0;
+  bool unfinished = true;
+  for (int its = 1; its <= 10 && unfinished; its++) {
+    p1 = 1.0;
+    p2 = 0.0;
+    for (int jj = 1; jj <= n; jj++) {
+      p3 = p2;
+      p2 = p1;
+      p1 = ((2.0 * jj - 1.0) * z * p2 - (jj - 1.0) * p3) / jj;
+    }
+    pp = n * (z * p1 - p2) / (z * z - 1.0);
+    z1 = z;
+    z = z1 - p1 / pp;
+    unfinished = fabs(z - z1) > 3.e-14;
+  }
+  // GauLeg writes x(j) then x(n-1-j); for the middle node of odd n the second wins
+  x = (k == n - 1 - j) ? xm + xl * z : xm - xl * z;
+  w = 2.0 * xl / ((1.0 - z * z) * pp * pp);
+}
+
+// node k of GauLeg_Sinh (common/ModQuadRule.F90:223-263)
+__device__ void sl_gauleg_sinh_node(double xmin, double xmax, double a, double b, int n, int k,
+                                 double &x, double &w) {
+  double xm = 0.5 * (xmin + xmax), xl = 0.5 * (xmax - xmin);
+  double a0 = (a - xm) / xl, b0 = b * xl;
+  double f1 = (1 + a0) / b0, f2 = (1 - a0) / b0;
+  double u1 = log(f1 + sqrt(1 + f1 * f1)), u2 = log(f2 + sqrt(1 + f2 * f2));
+  double mu = 0.5 * (u1 + u2), eta = 0.5 * (u1 - u2);
+  double sk, wk;
+  sl_gauleg_node(-1., 1., n, k, sk, wk);
+  double xk = a0 + b0 * sinh(mu * sk - eta);
+  wk = wk * b0 * mu * cosh(mu * sk - eta);
+  w = xl * wk;
+  x = xm + xl * xk;
+}
+
+__device__ void sl_readd_wave(const SingArgs &a, const CellRec &cr, const double *blk, int m, int n,
                            const double xi[3], const double x0[3], double th0, double phi0,
                            double radPat, double c1, double c2, double dv[3]) {
   const int nrad = 16, nazm = 32;
@@ -2382,9 +2522,9 @@ __device__ void readd_wave(const SingArgs &a, const CellRec &cr, const double *b
   double thl, wl;
   if (dist > 2.2250738585072014e-308) {
     dist = dist * (radPat / sizePat);
-    gauleg_sinh_node(0., radPat, 0., dist, nrad, irad, thl, wl);
+    sl_gauleg_sinh_node(0., radPat, 0., dist, nrad, irad, thl, wl);
   } else {
-    gauleg_node(0., radPat, nrad, irad, thl, wl);
+    sl_gauleg_node(0., radPat, nrad, irad, thl, wl);
   }
   double w = wl * sin(thl) * (RBC_TWO_PI / nazm);
   w = w * mask_fn(a.mtab, thl / radPat);
@@ -2441,10 +2581,7 @@ __device__ void readd_wave(const SingArgs &a, const CellRec &cr, const double *b
   dv[2] = wave_sum(a2);
 }
 
-// Near-singular stage 2: one wavefront per item that passed the distance test.
-// RBC_NearSingInt (:103-166) = subtract (:175-226) + re-add, or the interpolation
-// between the re-adds at xi1 and on the surface (with the double-layer jump).
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_near(SingArgs a, int nwork) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_near_sl(SingArgs a, int nwork) {
   int wid = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
   if (wid >= nwork) return;
   int it = a.work[2 * wid], cj = a.work[2 * wid + 1];
@@ -2537,13 +2674,159 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   }
   double dv[3] = {wave_sum(s0), wave_sum(s1), wave_sum(s2)}, dt[3];
   if (fabs(dist) >= fabs(dist1)) {
-    readd_wave(a, cr, blk, m, n, xi, x0, th0, phi0, radPat, c1, c2, dt);
+    sl_readd_wave(a, cr, blk, m, n, xi, x0, th0, phi0, radPat, c1, c2, dt);
     for (int d = 0; d < 3; d++) dv[d] += dt[d];
   } else {
     double xi1[3], dv1[3], dv0[3];
     for (int d = 0; d < 3; d++) xi1[d] = x0[d] + dist1 * a30[d];
-    readd_wave(a, cr, blk, m, n, xi1, x0, th0, phi0, radPat, c1, c2, dv1);
-    readd_wave(a, cr, blk, m, n, x0, x0, th0, phi0, radPat, c1, c2, dv0);
+    sl_readd_wave(a, cr, blk, m, n, xi1, x0, th0, phi0, radPat, c1, c2, dv1);
+    sl_readd_wave(a, cr, blk, m, n, x0, x0, th0, phi0, radPat, c1, c2, dv0);
+    if (c2 != 0) {
+      double detJ0, g0[3];
+      spline_interp(blk + vs * SPL_DETJ, m, n, th0, phi0, 1, &detJ0);
+      spline_interp(blk + vs * SPL_G, m, n, th0, phi0, 3, g0);
+      for (int d = 0; d < 3; d++) g0[d] = g0[d] / detJ0;
+      for (int d = 0; d < 3; d++) dv0[d] += (dist > 0 ? 1. : -1.) * c2 * 4 * RBC_PI * g0[d];
+    }
+    for (int d = 0; d < 3; d++) dv[d] += dv0[d] + dist / dist1 * (dv1[d] - dv0[d]);
+  }
+  if (lane == 0)
+    for (int d = 0; d < 3; d++) a.dvitem[3 * (size_t)it + d] = dv[d];
+}
+
+// Near-singular stage 2: one wavefront per item that passed the distance test.  Bound by
+// VALU issue (FP64 geometry and splines) and, close behind, by the address unit's rate on the
+// splines' scattered 16-byte loads; the registers limit the wavefronts that hide either.
+// 512 cells of 17 x 34 nodes 1.17 -> 0.79 ms, 4096 mixed cells 25.5 -> 17.5 ms, by walking
+// only the patch's nodes, the quadrature's roots from a table, and the item's values in
+// scalar registers, which leaves room for 3 wavefronts a SIMD (2: 0.94 ms, 4: 0.86 ms).
+// RBC_NearSingInt (:103-166) = subtract (:175-226) + re-add, or the interpolation
+// between the re-adds at xi1 and on the surface (with the double-layer jump).
+template <bool SL>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_near(SingArgs a, int nwork) {
+  // the item's values are the same in all lanes: told so, the compiler keeps them in
+  // scalar registers
+  const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
+  if (wid >= nwork) return;
+  const int it = __builtin_amdgcn_readfirstlane(a.work[2 * wid]);
+  const int cj = __builtin_amdgcn_readfirstlane(a.work[2 * wid + 1]);
+  const CellRec cr = a.cells[cj];
+  int gt = cr.gtype, m = 2 * cr.nlat, n = cr.nlon, nl = cr.nlat, nn = cr.nlon;
+  const double *r = a.item_rec + 12 * (size_t)it;
+  double xi[3] = {r[0], r[1], r[2]}, x0[3] = {r[3], r[4], r[5]}, a30[3] = {r[8], r[9], r[10]};
+  double th0 = r[6], phi0 = r[7], dist = r[11];
+  double radPat = cr.radius;
+  double c1 = a.c1, c2 = a.c2 * cr.Bcoef;
+  if (!SL && c2 == 0) {
+    if (lane < 3) a.dvitem[3 * (size_t)it + lane] = 0.;
+    return;
+  }
+  const double *blk = a.spl + cr.spl;
+  size_t vs = (size_t)m * n * 4;
+  double sizePat = radPat * sqrt(cr.area / (4 * RBC_PI));
+  double dist1 = copysign(0.01 * sizePat, dist);
+  // subtract: nodes of PolarPatch_FindPoints (common/ModPolarPatch.F90:161-209), with
+  // their multiplicity when the longitude range wraps more than once
+  const double *th = a.th[gt], *ph = a.phi[gt];
+  const double eps = 1.e-10;
+  double h_phi = RBC_TWO_PI / nn, ih_phi = 1.0 / h_phi, cosr0 = cos(radPat);
+  double s0 = 0, s1 = 0, s2 = 0;
+  // the longitude range of each latitude row inside the patch depends on the row only:
+  // lane i computes row i's (jmin, jmax) once (0 rows: outside the latitude band), and
+  // the node loop reads it from the wavefront's slot in LDS
+  __shared__ int rowj[256 / 64][64][2];
+  __shared__ double rowsc[256 / 64][64][2];  // the row's parts of the node's distance on the sphere
+  const int wsl = (int)(threadIdx.x >> 6);
+  int cnt = 0;
+  if (lane < nl) {
+    const int i = lane;
+    int jmin = 1, jmax = 0;
+    if (!(th[i] <= th0 - radPat) && !(th[i] >= th0 + radPat)) {
+      double dth = th[i] - th0;
+      double dphi = 1. - (cos(dth) - cosr0) / ((sin(th[i]) + eps) * (sin(th0) + eps));
+      dphi = fmax(-1., fmin(1., dphi));
+      dphi = acos(dphi);
+      if (dphi > RBC_PI - eps) {
+        jmin = 1;
+        jmax = nn;
+      } else {
+        jmin = (int)ceil((phi0 - dphi - ph[0]) * ih_phi) + 1;
+        jmax = (int)floor((phi0 + dphi - ph[0]) * ih_phi) + 1;
+      }
+    } else {
+      jmin = 1;
+      jmax = -(1 << 29);  // no node of this row
+    }
+    // a row spans at most once around, and one longitude more by rounding
+    cnt = min(max(jmax - jmin + 1, 0), 2 * nn);
+    rowj[wsl][i][0] = jmin;
+    rowsc[wsl][i][0] = cos(th0 - th[i]);
+    rowsc[wsl][i][1] = sin(th0) * sin(th[i]);
+  }
+  int incl = cnt;  // nodes of the rows up to this lane's
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += u;
+  }
+  const int total = __builtin_amdgcn_readlane(incl, 63);
+  rowj[wsl][lane][1] = incl - cnt;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  // the rows' nodes one after the other, an occurrence each: about one node in seven of the
+  // grid lies in the patch, so walking the grid left most of the lanes idle
+#pragma nounroll
+  for (int p = lane; p < total; p += 64) {
+    int i = 0;
+    for (int b = 32; b > 0; b >>= 1)
+      if (rowj[wsl][i + b][1] <= p) i += b;
+    const int jl = wrap_idx(rowj[wsl][i][0] - 1 + p - rowj[wsl][i][1], nn);
+    const int node = cr.off + i + nl * jl;
+    size_t np = a.np;
+    double xx[3];
+    for (int d = 0; d < 3; d++) xx[d] = a.x[node + np * d] - xi[d];
+    double rr = sqrt(xx[0] * xx[0] + xx[1] * xx[1] + xx[2] * xx[2]);
+    if (rr > a.rc) continue;
+    // dist_on_sphere(th0, phi0, th[i], ph[jl])
+    double ds = rowsc[wsl][i][0] - rowsc[wsl][i][1] * (1. - cos(phi0 - ph[jl]));
+    ds = fmin(1., fmax(-1., ds));
+    double mask = mask_fn(a.mtab, acos(ds) / radPat);
+    if (SL && c1 != 0) {
+      double fj[3] = {a.fs[node], a.fs[node + np], a.fs[node + 2 * np]}, EA, EB;
+      ewald_sl(a.sl1, a.sl2, rr, a.reps, a.rc, EA, EB);
+      double xf = xx[0] * fj[0] + xx[1] * fj[1] + xx[2] * fj[2];
+      s0 -= c1 * mask * (EA * xx[0] * xf + EB * fj[0]);
+      s1 -= c1 * mask * (EA * xx[1] * xf + EB * fj[1]);
+      s2 -= c1 * mask * (EA * xx[2] * xf + EB * fj[2]);
+    }
+    if (c2 != 0) {
+      double gj[3] = {a.gs[node], a.gs[node + np], a.gs[node + 2 * np]};
+      double nj[3] = {a.a3[node], a.a3[node + np], a.a3[node + 2 * np]};
+      double EA = ewald_dl(a.dl1, rr, a.reps, a.rc);
+      double xg = xx[0] * gj[0] + xx[1] * gj[1] + xx[2] * gj[2];
+      double xn = xx[0] * nj[0] + xx[1] * nj[1] + xx[2] * nj[2];
+      s0 -= c2 * mask * (EA * xx[0] * xg * xn);
+      s1 -= c2 * mask * (EA * xx[1] * xg * xn);
+      s2 -= c2 * mask * (EA * xx[2] * xg * xn);
+    }
+  }
+  double dv[3] = {wave_sum(s0), wave_sum(s1), wave_sum(s2)};
+  const bool apart = fabs(dist) >= fabs(dist1);
+  double dt[3], dv1[3] = {0, 0, 0};
+  // at the target itself, or at dist1 from the surface and then on it
+#pragma nounroll
+  for (int e = apart ? 1 : 0; e < 2; e++) {
+    double xe[3];
+    for (int d = 0; d < 3; d++) xe[d] = e == 0 ? x0[d] + dist1 * a30[d] : apart ? xi[d] : x0[d];
+    readd_wave<SL>(a, cr, blk, m, n, xe, x0, th0, phi0, radPat, c1, c2, dt);
+    if (e == 0)
+      for (int d = 0; d < 3; d++) dv1[d] = dt[d];
+  }
+  if (apart) {
+    for (int d = 0; d < 3; d++) dv[d] += dt[d];
+  } else {
+    double dv0[3] = {dt[0], dt[1], dt[2]};
     if (c2 != 0) {
       double detJ0, g0[3];
       spline_interp(blk + vs * SPL_DETJ, m, n, th0, phi0, 1, &detJ0);
@@ -3005,6 +3288,7 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   sa.gs = c->d_gs.p;
   sa.a3 = c->d_a3.p;
   sa.detj = c->d_detj.p;
+  sa.gl16 = c->d_gl16.p;
   sa.w_unused = nullptr;
   sa.tx = d_tx;
   sa.tA = d_A;
@@ -3049,12 +3333,21 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   }
   rbc_stage_end(c, ST_SELF);
   HIP_TRY(hipGetLastError());
+  auto near = [&](int nwork) {
+    const unsigned grid = (unsigned)(((size_t)nwork * 64 + 255) / 256);
+    if (c2 == 0 || !rbc_any_double_layer(c))
+      k_near_sl<<<grid, 256, 0, st>>>(sa, nwork);
+    else if (c1 != 0)
+      k_near<true><<<grid, 256, 0, st>>>(sa, nwork);
+    else
+      k_near<false><<<grid, 256, 0, st>>>(sa, nwork);
+  };
   if (nitems > 0 && hit) {
     const int nwork = c->cache_nwork;
     c->last_nwork = nwork;
     if (nwork > 0) {
       rbc_stage_begin(c, ST_NEAR);
-      k_near<<<(unsigned)(((size_t)nwork * 64 + 255) / 256), 256, 0, st>>>(sa, nwork);
+      near(nwork);
       rbc_stage_end(c, ST_NEAR);
       HIP_TRY(hipGetLastError());
     }
@@ -3087,7 +3380,7 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
     c->last_nwork = nwork;
     if (nwork > 0) {
       rbc_stage_begin(c, ST_NEAR);
-      k_near<<<(unsigned)(((size_t)nwork * 64 + 255) / 256), 256, 0, st>>>(sa, nwork);
+      near(nwork);
       rbc_stage_end(c, ST_NEAR);
       HIP_TRY(hipGetLastError());
     }
