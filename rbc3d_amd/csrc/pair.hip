@@ -1882,7 +1882,7 @@ __device__ __forceinline__ void nbr_sweep(const NbrArgs &a, const char *x0, cons
 // within twice the sweep's error bound of its smallest distance (nearly always one) are
 // evaluated in FP64, reduced by (distance, visit key, node).  Cells enter the list in
 // increasing index order.
-// What bounds it: VALU issue (about 15 cells within reach of a target), with the loads of
+// What bounds it: VALU issue (about 11 cells within reach of a target), with the loads of
 // the sweep close behind.  The FP64 sweep behind bounding spheres of 64-node strips that
 // was here took some 600 instructions a cell.  296k targets on 512 cells 4.54 -> 1.33
 // ms; on 4096 cells of mixed grids 17.0 -> 5.4 ms; 20,000 points among 128 cells 353 -> 104 us.
