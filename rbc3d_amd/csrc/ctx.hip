@@ -598,8 +598,9 @@ extern "C" int rbc3d_destroy(rbc3d_ctx *c) {
                        &c->d_torder, &c->d_tbin_start, &c->d_chunk_off, &c->d_clus, &c->d_nbr_cnt,
                        &c->d_nbr_cell, &c->d_nbr_node, &c->d_cell_cand, &c->d_work, &c->d_work_cnt, &c->d_flag,
                        &c->d_cellbin_start, &c->d_cellbin_order, &c->d_pme_key, &c->d_pme_order,
-                       &c->d_pme_start, &c->wall.d_e2v, &c->wall.d_glb, &c->wall.d_bin_start,
-                       &c->wall.d_order, &c->wall.d_rowptr, &c->wall.d_col})
+                       &c->d_pme_start, &c->spread_sort[0].order, &c->spread_sort[0].start,
+                       &c->spread_sort[1].order, &c->spread_sort[1].start, &c->wall.d_e2v,
+                       &c->wall.d_glb, &c->wall.d_bin_start, &c->wall.d_order, &c->wall.d_rowptr, &c->wall.d_col})
     b->release();
   c->d_cells.release();
   c->d_cub_tmp.release();

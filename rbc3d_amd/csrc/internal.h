@@ -290,9 +290,15 @@ struct rbc3d_ctx {
   GmresWork gmres;
   DBuf<double> d_linpart;
   unsigned long long last_checksum = 0;
-  // the PME spread's sort of the cell sources by brick depends on the geometry only:
-  // kept for the geometry epoch it was made at (with geometry reuse on)
-  int spread_sort_epoch = -1, spread_sort_ns = 0, spread_sort_edge = 0;
+  // the PME spread's sorts of the cell sources by brick depend on the geometry only: with
+  // geometry reuse on, one for each brick edge is kept in buffers of its own for the
+  // geometry epoch it was made at.  Nothing else writes them, so a recorded matvec, which
+  // holds the buffers and not the sort, may be replayed after a call that sorts otherwise
+  // (the right-hand side, a sum over cells and walls).
+  struct SpreadSort {
+    int epoch = -1, ns = 0;
+    DBuf<int> order, start;
+  } spread_sort[2];
   // hipGraph of the cell matvec at fixed geometry (rbc3d_set_graph): captured on the
   // matvec's own input and output buffers, valid for one geometry epoch, precision
   // form and buffer-allocation count

@@ -832,9 +832,17 @@ static int pme_spread_t(rbc3d_ctx *c, double c1, double c2, int cells, int walls
   RBC_TRY(c->d_pme_src.ensure((size_t)reclen * ns + 1));
   RBC_TRY(c->d_pme_key.ensure(2 * (size_t)ns + 2));
   RBC_TRY(c->d_pme_order.ensure(2 * (size_t)ns + 2));
-  RBC_TRY(c->d_pme_start.ensure(nbr + 1));
+  // The sources' order by brick depends on the positions only: with geometry reuse, the
+  // cell sources' sort (order, brick starts) is kept for the geometry epoch it was made
+  // at, one for each brick edge; a sort with wall elements goes to the shared buffers.
+  const bool keep = cells && !walls && ncell > 0 && c->geom_reuse;
+  auto &kept = c->spread_sort[bricks];
+  const bool sorted = keep && kept.epoch == c->geom_epoch && kept.ns == ns;
+  DBuf<int> &start = keep ? kept.start : c->d_pme_start;
+  RBC_TRY(start.ensure(nbr + 1));
+  if (keep) RBC_TRY(kept.order.ensure(ns));
   int *key = c->d_pme_key.p, *key2 = c->d_pme_key.p + ns + 1;
-  int *idx = c->d_pme_order.p + ns + 1, *order = c->d_pme_order.p;
+  int *idx = c->d_pme_order.p + ns + 1, *order = keep ? kept.order.p : c->d_pme_order.p;
   if (ns > 0) {
     rbc_stage_begin(c, ST_SPREAD_PREP);
     k_spread_prep<T><<<(ns + 255) / 256, 256, 0, st>>>(
@@ -845,13 +853,8 @@ static int pme_spread_t(rbc3d_ctx *c, double c1, double c2, int cells, int walls
     rbc_stage_end(c, ST_SPREAD_PREP);
     HIP_TRY(hipGetLastError());
   }
-  // The sources' order by brick depends on the positions only: with geometry reuse, the
-  // cell sources' sort (order, brick starts) is kept for the geometry epoch it was made
-  // at.  Every call that sorts replaces it, so the kept one is the last sort made.
-  const bool keep = cells && !walls && ncell > 0 && c->geom_reuse;
-  const bool sorted = keep && c->spread_sort_epoch == c->geom_epoch && c->spread_sort_ns == ns &&
-                      c->spread_sort_edge == edge;
   if (!sorted) {
+    if (keep) kept.epoch = -1;
     if (ns > 0) {
       int bits = 1;
       while ((1 << bits) < nbr) bits++;
@@ -861,12 +864,13 @@ static int pme_spread_t(rbc3d_ctx *c, double c1, double c2, int cells, int walls
       HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->d_cub_tmp.p, tmp, key, key2, idx, order, ns, 0,
                                                  bits, st));
     }
-    k_brick_start<<<(nbr + 1 + 255) / 256, 256, 0, st>>>(ns, key2, nbr, c->d_pme_start.p);
+    k_brick_start<<<(nbr + 1 + 255) / 256, 256, 0, st>>>(ns, key2, nbr, start.p);
     HIP_TRY(hipGetLastError());
+    if (keep) {
+      kept.epoch = c->geom_epoch;
+      kept.ns = ns;
+    }
   }
-  c->spread_sort_epoch = keep ? c->geom_epoch : -1;
-  c->spread_sort_ns = ns;
-  c->spread_sort_edge = edge;
   SpreadArgs<T> a;
   a.N1 = N1;
   a.N2 = N2;
@@ -883,7 +887,7 @@ static int pme_spread_t(rbc3d_ctx *c, double c1, double c2, int cells, int walls
   a.flag_dl = c->flag_dl;
   a.rec = (const T *)c->d_pme_src.p;
   a.order = order;
-  a.brick_start = c->d_pme_start.p;
+  a.brick_start = start.p;
   a.grid = (T *)c->d_grid.p;
   if (P > 12) {
     rbc_set_error("B-spline order above 12");

@@ -97,3 +97,35 @@ def test_graph_off_without_geometry_reuse(mixed):
     finally:
         g.set_graph(False)
         g.set_geometry_reuse(True)
+
+
+@pytest.mark.parametrize("name", ["C5", "C3s"])
+def test_replays_after_other_sums(name):
+    """Replays after calls that sort the sources in another way than the recorded matvec (the
+    right-hand side, the single layer alone, cells and walls together): bit for bit the
+    eager matvec.  A suspension, and cells in a tube."""
+    import torch
+    import rbc3d_amd
+    from rbc3d_amd import configs
+    w = configs.make_workload(name, seed=1, **(dict(ncell=16, Nb=(32, 32, 32)) if name == "C5" else {}))
+    w.viscRat = (5.0,) * len(w.viscRat)
+    g = rbc3d_amd.from_workload(w)
+    if w.wall is not None:
+        g.prepare_sing_int_on_wall()
+    tl = g.tlist_rbc()
+    others = {"rhs": g.cell_rhs, "single": lambda: g.pme(1.0, 0.0, tl, walls=False),
+              "both": lambda: g.pme(1.0, 1.0, tl, walls=False), "walls": lambda: g.pme(1.0, 1.0, tl)}
+    us = [torch.randn(g.cell_dof(), dtype=torch.float64, device="cuda",
+                      generator=torch.Generator(device="cuda").manual_seed(k)) for k in range(2)]
+    g.set_geometry_reuse(True)
+    for prec in (g.PREC_FP64, g.PREC_SPLIT):
+        ref = _eager(g, us, prec)
+        values = {k: f() for k, f in others.items()}
+        g.set_graph(True)
+        _replays(g, us, ref, f"{name}, precision {prec}")
+        for _ in range(2):
+            for k, f in others.items():
+                assert (f() == values[k]).all(), k
+                g.sync()
+                _replays(g, us, ref, f"{name}, precision {prec}, after {k}")
+    g.close()
