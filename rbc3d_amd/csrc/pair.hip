@@ -727,7 +727,9 @@ __global__ void __launch_bounds__(64 * (SL ? 12 : 16)) k_pair(PairArgs a) {
       // The cluster's bounding sphere over its active targets, each taken back into the
       // box (x - kt Lb): a candidate whose image (or minimum image) is farther than
       // rc + r (plus a margin far above the roundings) from the centre is beyond rc of
-      // every target.  All slots hold the same targets.
+      // every target.  All slots hold the same targets.  A cluster with a target thousands
+      // of periods away, whose place in the box has lost digits (or whose bin numbers do not
+      // fit 32 bits), keeps every candidate instead.
       double ct0, ct1, ct2, cut;
       {
         const double w0 = act ? xi0 - kt0 * L0 : 0., w1 = act ? xi1 - kt1 * L1 : 0.,
@@ -748,6 +750,10 @@ __global__ void __launch_bounds__(64 * (SL ? 12 : 16)) k_pair(PairArgs a) {
 #pragma unroll
         for (int o = PC / 2; o > 0; o >>= 1) r2 = fmax(r2, __shfl_xor(r2, o, 64));
         cut = wave_uniform(a.rc * (1. + 1e-9) + sqrt(r2) + 1e-9 * (1. + L0 + L1 + L2));
+        if (__ballot(act && max(abs(kt0), max(abs(kt1), abs(kt2))) > 4096) != 0ull) {
+          ct0 = ct1 = ct2 = 0.;
+          cut = 4. * (L0 + L1 + L2);
+        }
         ct0 = wave_uniform(ct0);
         ct1 = wave_uniform(ct1);
         ct2 = wave_uniform(ct2);

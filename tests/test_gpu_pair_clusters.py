@@ -61,3 +61,29 @@ def test_viscosity_ratio_one():
         vg = g.add_int_on_rbcs(c1, c2, tl)
         assert g.pair_stats()[0] == npairs
         assert np.abs(vg - vo).max() <= TOL * max(np.abs(vo).max(), 1.0)
+
+
+@pytest.mark.parametrize("L", [13.0, 5.0])
+def test_far_targets(L):
+    """Points so many periods away that their bins' numbers leave 32 bits, in one cluster with
+    points in the box: these keep their velocities."""
+    import rbc3d_amd as R
+    w = suspension(L, 6 if L > 8 else 1, 11, False)
+    g, o = R.from_workload(w), O.from_workload(w)
+    rng = np.random.default_rng(2)
+    Nf = 2 * max(int(L // w.rc), 3)
+    bins = np.array([(2**31 - 1) % Nf, (-2**31) % Nf])  # the bins that such points fall in
+    near = ((bins[:, None, None] + rng.random((2, 7, 3))) * L / Nf).reshape(-1, 3)
+    pts = np.concatenate([near, [[1e13] * 3, [-1e13] * 3]])
+
+    def tl(p):
+        k = len(p)
+        return p.reshape(-1, order="F").copy(), np.zeros(3 * k, np.int32), np.ones(k, np.int32), np.ones(k)
+
+    for c1, c2 in ((0.0, 1.0), (0.7, -1.3)):
+        vo = o.add_int_on_rbcs(c1, c2, tl(near))[0].reshape(3, -1)
+        vg = g.add_int_on_rbcs(c1, c2, tl(pts)).reshape(3, -1)[:, :len(near)]
+        assert np.abs(vo).max() > 0
+        err = np.abs(vg - vo).max() / np.abs(vo).max()
+        print(f"box {L}, {c1}, {c2}: {err:.2e}", flush=True)
+        assert err < TOL
