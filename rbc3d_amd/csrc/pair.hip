@@ -2247,6 +2247,13 @@ __global__ void __launch_bounds__(SELF_T) k_self_own(SelfArgs a) {
   const CellRec cr = a.cells[rl.x];
   const int gt = cr.gtype, m = 2 * cr.nlat, n = cr.nlon, ilat = rl.y;
   const int npt = a.nrad[gt] * a.nazm[gt], nrad = a.nrad[gt], nb = a.nband[gt], r0 = a.rows[gt][ilat];
+  const double c2m = a.c2 * cr.Bcoef;
+  if (c2m == 0.) {  // no double layer on this cell
+    if ((int)threadIdx.x < n)
+      for (int d = 0; d < 3; d++)
+        a.dvself[cr.off + ilat + cr.nlat * (int)threadIdx.x + (size_t)a.nT * d] = 0.;
+    return;
+  }
   const double *blk = a.spl + cr.spl;
   const size_t vs = (size_t)m * n * 4;
   // the band: row r0 + i at i, all longitudes
@@ -2316,12 +2323,11 @@ __global__ void __launch_bounds__(SELF_T) k_self_own(SelfArgs a) {
   red[2][threadIdx.x] = dv2;
   __syncthreads();
   if ((int)threadIdx.x < n) {
-    const double c2m = a.c2 * cr.Bcoef;
     const int ti = cr.off + ilat + cr.nlat * (int)threadIdx.x;
     for (int d = 0; d < 3; d++) {
       double v = red[d][threadIdx.x];
       for (int g = 1; g < ngrp; g++) v += red[d][g * n + threadIdx.x];
-      a.dvself[ti + (size_t)a.nT * d] = c2m != 0 ? c2m * v : 0.;
+      a.dvself[ti + (size_t)a.nT * d] = c2m * v;
     }
   }
 }
