@@ -1,4 +1,4 @@
-"""The network's training kernel at the edges of its split (tiles of 16 nodes, four
+"""The network's training kernel at the edges of its split (tiles of 16 nodes, up to four
 wavefronts a workgroup, at most 256 workgroups) and its GELU far from zero, against the
 CPU oracle."""
 import numpy as np
@@ -10,7 +10,7 @@ from tests.test_gpu_mlp import _data, _net
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 16384, 16401])
+@pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 4096, 4097, 16384, 16401])
 def test_gradient_batches(n):
     import torch
     import rbc3d_amd as R
