@@ -54,6 +54,7 @@ enum { SW_1 = 0, SW_2 = SW_1 + 64 * MLP_TS1, SW_3 = SW_2 + 64 * MLP_TS, SW_4 = S
        SW_N = SW_4 + 16 * MLP_TS,
        ST_2 = SW_N, ST_3 = ST_2 + 64 * MLP_TS, ST_4 = ST_3 + 64 * MLP_TS, ST_N = ST_4 + 64 * MLP_TS1 };
 #define MLP_TW 4   // wavefronts per training workgroup
+#define MLP_WG (64 * MLP_TW)  // threads of the forward's and the training's workgroups
 // LDS copies of the biases b1 b2 b3 (64 each), b4 (3) and the norm
 enum { SB_4 = 3 * 64, SB_NORM = SB_4 + 4, SB_N = SB_NORM + 2 * MLP_NIN + MLP_NOUT };
 
@@ -192,7 +193,7 @@ __device__ __forceinline__ void load_biases(float *sb, const float *p, const flo
 __device__ __forceinline__ void load_weights(unsigned short *sW, const unsigned short *wb, bool tr) {
   static_assert(WB_N % 4 == 0, "four weights at a time");
   #pragma unroll 5
-  for (int t4 = threadIdx.x; t4 < WB_N / 4; t4 += 256) {
+  for (int t4 = threadIdx.x; t4 < WB_N / 4; t4 += MLP_WG) {
     const mlp_s4 v = reinterpret_cast<const mlp_s4 *>(wb)[t4];
     const int t = 4 * t4;
     if (t < WB_2) {
@@ -210,7 +211,7 @@ __device__ __forceinline__ void load_weights(unsigned short *sW, const unsigned 
 }
 
 // inference: Y[node][c] = scale_c * y_c (the predicted traction increment)
-__global__ void __launch_bounds__(256) k_mlp_forward(int n, const float *__restrict__ X,
+__global__ void __launch_bounds__(MLP_WG) k_mlp_forward(int n, const float *__restrict__ X,
                                                      const unsigned short *__restrict__ wb,
                                                      const float *__restrict__ p,
                                                      const float *__restrict__ norm, float *Y) {
@@ -302,7 +303,7 @@ __device__ __forceinline__ void put_bias(float *red, mlp_f4 v, int lane, bool fi
 // all its sums in registers (160 of them matrix accumulators, one wavefront a SIMD): in
 // LDS, where every tile's products were added before, a tile cost 640 more LDS accesses
 // and 200 lane exchanges for the biases.  65,536 rows: 135 -> 58 us.
-__global__ void __launch_bounds__(64 * MLP_TW, 1) k_mlp_train(int n, const float *__restrict__ X,
+__global__ void __launch_bounds__(MLP_WG, 1) k_mlp_train(int n, const float *__restrict__ X,
                                                   const float *__restrict__ Tg,
                                                   const unsigned short *__restrict__ wb,
                                                   const float *__restrict__ p,
@@ -415,7 +416,7 @@ __global__ void __launch_bounds__(64 * MLP_TW, 1) k_mlp_train(int n, const float
     }
     __syncthreads();
   }
-  for (int t = threadIdx.x; t < GA_N; t += 64 * MLP_TW) part[(size_t)blockIdx.x * GA_N + t] = red[t];
+  for (int t = threadIdx.x; t < GA_N; t += MLP_WG) part[(size_t)blockIdx.x * GA_N + t] = red[t];
   if (threadIdx.x == 0) {
     double s = 0.;
     for (int w = 0; w < MLP_TW; w++) s += lred[w];
@@ -589,7 +590,7 @@ int rbc_mlp_forward(rbc3d_mlp *m, int n, const float *d_x, float *d_y, hipStream
   if (n <= 0) return RBC3D_OK;
   const int ntile = (n + 15) / 16;
   const unsigned nblk = (unsigned)std::min(1024, (ntile + 3) / 4);
-  k_mlp_forward<<<nblk, 256, 0, st>>>(n, d_x, m->wb.p, m->p.p, m->norm.p, d_y);
+  k_mlp_forward<<<nblk, MLP_WG, 0, st>>>(n, d_x, m->wb.p, m->p.p, m->norm.p, d_y);
   HIP_TRY(hipGetLastError());
   return RBC3D_OK;
 }
@@ -610,7 +611,7 @@ static int mlp_grad(rbc3d_mlp *m, int n, const float *d_x, const float *d_t, dou
   const int nwg = std::min(256, ntile);
   RBC_TRY(m->part.ensure((size_t)nwg * GA_N));
   RBC_TRY(m->lpart.ensure(nwg));
-  k_mlp_train<<<nwg, 64 * MLP_TW, 0, m->st()>>>(n, d_x, d_t, m->wb.p, m->p.p, m->norm.p,
+  k_mlp_train<<<nwg, MLP_WG, 0, m->st()>>>(n, d_x, d_t, m->wb.p, m->p.p, m->norm.p,
                                                 m->part.p, m->lpart.p);
   k_mlp_reduce<<<(MP_N + 63) / 64, 64 * MLP_RW, 0, m->st()>>>(nwg, m->part.p, m->grad.p);
   HIP_TRY(hipGetLastError());
