@@ -525,7 +525,7 @@ struct PairArgs {
   double Lb[3], iLb[3], iLbNf[3], w[3];  // box, 1/box, 1/bin width, bin width
   int Nf[3];
   int img;  // 1: periodic images from the visited bins (every dimension has >= 2R+3 bins)
-  double rc, rc2, rc2hi, rc2lo, rc2w, reps2, tabscale, c1, c2;  // rc2w: half width of the shell
+  double rc, rc2hi, rc2lo, reps2, tabscale, c1, c2;
   int np, nT, nfbins, nrbc, nrows;
   const int *rows;       // x-rows of source bins: packed (alo, ahi, o2, o3)
   const double *rec;     // sources sorted by fine bin (SREC x np)
@@ -3147,9 +3147,7 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   }
   pa.img = c->pair_img;
   pa.rc = c->conf.rc;
-  pa.rc2 = c->conf.rc * c->conf.rc;
   pa.rc2hi = c->conf.rc * c->conf.rc * (1.0 + 1e-12);
-  pa.rc2w = c->conf.rc * c->conf.rc * 2e-12;
   pa.rc2lo = c->conf.rc * c->conf.rc * (1.0 - 1e-12);
   pa.reps2 = c->r_eps * c->r_eps;
   pa.tabscale = RBC_NTAB / c->conf.rc;
