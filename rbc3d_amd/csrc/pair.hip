@@ -2399,8 +2399,32 @@ __global__ void k_items(int nT, const int *__restrict__ cnt, const int *__restri
   }
 }
 
+// The single layer's sums of the near-singular correction are written with their
+// contractions: they enter the walls' velocities, whose solver's iteration count hangs on
+// their last bits (traction to 1e-5), so they must not follow what the compiler makes of the
+// code around them.  FS: the table's fractions i + 1 - r K and r K - i in one rounding each.
+// (tests/golden/single_layer_near.npz holds the path's values, geometry included.)
+__device__ __forceinline__ double dot3(const double a[3], const double b[3]) {
+#pragma clang fp contract(off)
+  return fma(a[2], b[2], fma(a[0], b[0], a[1] * b[1]));
+}
+template <bool FS>
+__device__ __forceinline__ void ewald_sl_near(const SingArgs &a, double r, double &A, double &B) {
+#pragma clang fp contract(off)
+  A = B = 0.;
+  if (r < a.reps) return;
+  const double K = RBC_NTAB / a.rc, s = r * K, fi = floor(s);
+  if (fi >= RBC_NTAB) return;
+  const int i = (int)fi;
+  const double w0 = FS ? fma(-K, r, i + 1) : i + 1 - s, w1 = FS ? fma(K, r, -i) : s - i;
+  const double c1 = fma(w0, a.sl1[i], w1 * a.sl1[i + 1]), c2 = fma(w0, a.sl2[i], w1 * a.sl2[i + 1]);
+  const double ir = rcp_nr(r), ir2 = ir * ir;
+  A = fma(ir2, ir * c1, ir2 * c2);
+  B = fma(ir, c1, -c2);
+}
+
 // RBC_NearSingInt_ReAdd (common/ModRbcSingInt.F90:232-310), lanes over the 16 x 32 patch
-template <bool SL>
+template <bool SL, bool DL>
 __device__ __forceinline__ void readd_wave(const SingArgs &a, const CellRec &cr, const double *blk, int m, int n,
                            const double xi[3], const double x0[3], double th0, double phi0,
                            double radPat, double c1, double c2, double dv[3]) {
@@ -2408,8 +2432,8 @@ __device__ __forceinline__ void readd_wave(const SingArgs &a, const CellRec &cr,
   // lane l always takes radial node l % 16 (64 is a multiple of nrad): its node and
   // masked weight are computed once
   const int lane = threadIdx.x & 63, irad = lane & (nrad - 1);
-  double d0 = xi[0] - x0[0], d1 = xi[1] - x0[1], d2 = xi[2] - x0[2];
-  double dist = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+  const double d[3] = {xi[0] - x0[0], xi[1] - x0[1], xi[2] - x0[2]};
+  double dist = sqrt(dot3(d, d));
   double sizePat = radPat * sqrt(cr.area / (4 * RBC_PI));
   double thl, wl;
   if (dist > 2.2250738585072014e-308) {
@@ -2444,19 +2468,20 @@ __device__ __forceinline__ void readd_wave(const SingArgs &a, const CellRec &cr,
     double xj[3], xx[3];
     spline_interp(blk + vs * SPL_X, m, n, thj, phj, 3, xj);
     for (int d = 0; d < 3; d++) xx[d] = xj[d] - xi[d];
-    double rr = sqrt(xx[0] * xx[0] + xx[1] * xx[1] + xx[2] * xx[2]);
+    const double rr = sqrt(dot3(xx, xx));
     if (rr > a.rc) continue;
     if (SL && c1 != 0) {
+#pragma clang fp contract(off)
       double fj[3], EA, EB;
       spline_interp(blk + vs * SPL_F, m, n, thj, phj, 3, fj);
       for (int d = 0; d < 3; d++) fj[d] = w * fj[d];
-      ewald_sl(a.sl1, a.sl2, rr, a.reps, a.rc, EA, EB);
-      double xf = xx[0] * fj[0] + xx[1] * fj[1] + xx[2] * fj[2];
-      a0 += c1 * (EA * xx[0] * xf + EB * fj[0]);
-      a1 += c1 * (EA * xx[1] * xf + EB * fj[1]);
-      a2 += c1 * (EA * xx[2] * xf + EB * fj[2]);
+      ewald_sl_near<false>(a, rr, EA, EB);
+      const double xf = dot3(xx, fj);
+      a0 = fma(c1, fma(fj[0], EB, EA * xx[0] * xf), a0);
+      a1 = fma(c1, fma(fj[1], EB, EA * xx[1] * xf), a1);
+      a2 = fma(c1, fma(fj[2], EB, EA * xx[2] * xf), a2);
     }
-    if (c2 != 0) {
+    if (DL && c2 != 0) {
       double gj[3], nj[3];
       spline_interp(blk + vs * SPL_A3, m, n, thj, phj, 3, nj);
       spline_interp(blk + vs * SPL_G, m, n, thj, phj, 3, gj);
@@ -2474,125 +2499,9 @@ __device__ __forceinline__ void readd_wave(const SingArgs &a, const CellRec &cr,
   dv[2] = wave_sum(a2);
 }
 
-// The near-singular correction of calls without a double layer, in the order that it has
-// always summed in: its results enter the walls' velocities, whose solver's iteration count
-// hangs on their last bits (traction to 1e-5), so this path keeps every operation.  The
-// double-layer terms below are never taken here, but without them the compiler contracts
-// the others differently (measured: 3% of the results change in the last bit).
-// GauLeg (common/ModQuadRule.F90:135-208), node k (ascending) and its weight: each root's Newton iteration is
-// independent of the others, so one lane computes one node, as GauLeg does for it.
-__device__ void sl_gauleg_node(double x1, double x2, int n, int k, double &x, double &w) {
-  const int m = (n + 1) / 2;
-  const int j = k < m ? k : n - 1 - k;
-  double xm = 0.5 * (x2 + x1), xl = 0.5 * (x2 - x1);
-  double z = cos(RBC_PI * ((j + 1) - 0.25) / (n + 0.5)), z1, p1 = 0, p2, p3, pp = 0;
-  bool unfinished = true;
-  for (int its = 1; its <= 10 && unfinished; its++) {
-    p1 = 1.0;
-    p2 = 0.0;
-    for (int jj = 1; jj <= n; jj++) {
-      p3 = p2;
-      p2 = p1;
-      p1 = ((2.0 * jj - 1.0) * z * p2 - (jj - 1.0) * p3) / jj;
-    }
-    pp = n * (z * p1 - p2) / (z * z - 1.0);
-    z1 = z;
-    z = z1 - p1 / pp;
-    unfinished = fabs(z - z1) > 3.e-14;
-  }
-  // GauLeg writes x(j) then x(n-1-j); for the middle node of odd n the second wins
-  x = (k == n - 1 - j) ? xm + xl * z : xm - xl * z;
-  w = 2.0 * xl / ((1.0 - z * z) * pp * pp);
-}
-
-// node k of GauLeg_Sinh (common/ModQuadRule.F90:223-263)
-__device__ void sl_gauleg_sinh_node(double xmin, double xmax, double a, double b, int n, int k,
-                                 double &x, double &w) {
-  double xm = 0.5 * (xmin + xmax), xl = 0.5 * (xmax - xmin);
-  double a0 = (a - xm) / xl, b0 = b * xl;
-  double f1 = (1 + a0) / b0, f2 = (1 - a0) / b0;
-  double u1 = log(f1 + sqrt(1 + f1 * f1)), u2 = log(f2 + sqrt(1 + f2 * f2));
-  double mu = 0.5 * (u1 + u2), eta = 0.5 * (u1 - u2);
-  double sk, wk;
-  sl_gauleg_node(-1., 1., n, k, sk, wk);
-  double xk = a0 + b0 * sinh(mu * sk - eta);
-  wk = wk * b0 * mu * cosh(mu * sk - eta);
-  w = xl * wk;
-  x = xm + xl * xk;
-}
-
-__device__ void sl_readd_wave(const SingArgs &a, const CellRec &cr, const double *blk, int m, int n,
-                           const double xi[3], const double x0[3], double th0, double phi0,
-                           double radPat, double c1, double c2, double dv[3]) {
-  const int nrad = 16, nazm = 32;
-  // lane l always takes radial node l % 16 (64 is a multiple of nrad): its node and
-  // masked weight are computed once
-  const int lane = threadIdx.x & 63, irad = lane & (nrad - 1);
-  double d0 = xi[0] - x0[0], d1 = xi[1] - x0[1], d2 = xi[2] - x0[2];
-  double dist = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-  double sizePat = radPat * sqrt(cr.area / (4 * RBC_PI));
-  double thl, wl;
-  if (dist > 2.2250738585072014e-308) {
-    dist = dist * (radPat / sizePat);
-    sl_gauleg_sinh_node(0., radPat, 0., dist, nrad, irad, thl, wl);
-  } else {
-    sl_gauleg_node(0., radPat, nrad, irad, thl, wl);
-  }
-  double w = wl * sin(thl) * (RBC_TWO_PI / nazm);
-  w = w * mask_fn(a.mtab, thl / radPat);
-  size_t vs = (size_t)m * n * 4;
-  double s0 = sin(th0), c0 = cos(th0);
-  double a0 = 0, a1 = 0, a2 = 0;
-  // sin and cos of the nazm azimuths, once per wavefront (lane j < nazm: azimuth j, the
-  // same expression as the point loop's), and of the lane's own radial angle
-  __shared__ double azsc[256 / 64][nazm][2];
-  const int wsl = (int)(threadIdx.x >> 6);
-  if (lane < nazm) {
-    const double phL = lane * RBC_TWO_PI / nazm;
-    azsc[wsl][lane][0] = sin(phL);
-    azsc[wsl][lane][1] = cos(phL);
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  const double stl = sin(thl), ctl = cos(thl);
-  for (int p = lane; p < nrad * nazm; p += 64) {
-    int iazm = p / nrad;
-    double thj, phj;
-    patch_point_sc(s0, c0, phi0, stl, ctl, azsc[wsl][iazm][0], azsc[wsl][iazm][1], thj, phj);
-    double xj[3], xx[3];
-    spline_interp(blk + vs * SPL_X, m, n, thj, phj, 3, xj);
-    for (int d = 0; d < 3; d++) xx[d] = xj[d] - xi[d];
-    double rr = sqrt(xx[0] * xx[0] + xx[1] * xx[1] + xx[2] * xx[2]);
-    if (rr > a.rc) continue;
-    if (c1 != 0) {
-      double fj[3], EA, EB;
-      spline_interp(blk + vs * SPL_F, m, n, thj, phj, 3, fj);
-      for (int d = 0; d < 3; d++) fj[d] = w * fj[d];
-      ewald_sl(a.sl1, a.sl2, rr, a.reps, a.rc, EA, EB);
-      double xf = xx[0] * fj[0] + xx[1] * fj[1] + xx[2] * fj[2];
-      a0 += c1 * (EA * xx[0] * xf + EB * fj[0]);
-      a1 += c1 * (EA * xx[1] * xf + EB * fj[1]);
-      a2 += c1 * (EA * xx[2] * xf + EB * fj[2]);
-    }
-    if (c2 != 0) {
-      double gj[3], nj[3];
-      spline_interp(blk + vs * SPL_A3, m, n, thj, phj, 3, nj);
-      spline_interp(blk + vs * SPL_G, m, n, thj, phj, 3, gj);
-      for (int d = 0; d < 3; d++) gj[d] = w * gj[d];
-      double EA = ewald_dl(a.dl1, rr, a.reps, a.rc);
-      double xg = xx[0] * gj[0] + xx[1] * gj[1] + xx[2] * gj[2];
-      double xn = xx[0] * nj[0] + xx[1] * nj[1] + xx[2] * nj[2];
-      a0 += c2 * (EA * xx[0] * xg * xn);
-      a1 += c2 * (EA * xx[1] * xg * xn);
-      a2 += c2 * (EA * xx[2] * xg * xn);
-    }
-  }
-  dv[0] = wave_sum(a0);
-  dv[1] = wave_sum(a1);
-  dv[2] = wave_sum(a2);
-}
-
+// The near-singular correction of calls without a double layer: k_near (below) but for the
+// lanes' walk over the whole grid, the order that the single layer has always been summed
+// in and that the wall solves follow.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_near_sl(SingArgs a, int nwork) {
   int wid = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
   if (wid >= nwork) return;
@@ -2603,7 +2512,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   double xi[3] = {r[0], r[1], r[2]}, x0[3] = {r[3], r[4], r[5]}, a30[3] = {r[8], r[9], r[10]};
   double th0 = r[6], phi0 = r[7], dist = r[11];
   double radPat = cr.radius;
-  double c1 = a.c1, c2 = a.c2 * cr.Bcoef;
+  const double c1 = a.c1;
   const double *blk = a.spl + cr.spl;
   size_t vs = (size_t)m * n * 4;
   double sizePat = radPat * sqrt(cr.area / (4 * RBC_PI));
@@ -2659,48 +2568,32 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
     size_t np = a.np;
     double xx[3];
     for (int d = 0; d < 3; d++) xx[d] = a.x[node + np * d] - xi[d];
-    double rr = sqrt(xx[0] * xx[0] + xx[1] * xx[1] + xx[2] * xx[2]);
+    const double rr = sqrt(dot3(xx, xx));
     if (rr > a.rc) continue;
-    double dthm = dist_on_sphere(th0, phi0, th[i], ph[jl]);
-    double mask = mask_fn(a.mtab, dthm / radPat);
-    for (int rep = 0; rep < mult; rep++) {
-      if (c1 != 0) {
-        double fj[3] = {a.fs[node], a.fs[node + np], a.fs[node + 2 * np]}, EA, EB;
-        ewald_sl(a.sl1, a.sl2, rr, a.reps, a.rc, EA, EB);
-        double xf = xx[0] * fj[0] + xx[1] * fj[1] + xx[2] * fj[2];
-        s0 -= c1 * mask * (EA * xx[0] * xf + EB * fj[0]);
-        s1 -= c1 * mask * (EA * xx[1] * xf + EB * fj[1]);
-        s2 -= c1 * mask * (EA * xx[2] * xf + EB * fj[2]);
-      }
-      if (c2 != 0) {
-        double gj[3] = {a.gs[node], a.gs[node + np], a.gs[node + 2 * np]};
-        double nj[3] = {a.a3[node], a.a3[node + np], a.a3[node + 2 * np]};
-        double EA = ewald_dl(a.dl1, rr, a.reps, a.rc);
-        double xg = xx[0] * gj[0] + xx[1] * gj[1] + xx[2] * gj[2];
-        double xn = xx[0] * nj[0] + xx[1] * nj[1] + xx[2] * nj[2];
-        s0 -= c2 * mask * (EA * xx[0] * xg * xn);
-        s1 -= c2 * mask * (EA * xx[1] * xg * xn);
-        s2 -= c2 * mask * (EA * xx[2] * xg * xn);
+    const double mask = mask_fn(a.mtab, dist_on_sphere(th0, phi0, th[i], ph[jl]) / radPat);
+    {
+#pragma clang fp contract(off)
+      const double fj[3] = {a.fs[node], a.fs[node + np], a.fs[node + 2 * np]}, cm = c1 * mask;
+      double EA, EB;
+      ewald_sl_near<true>(a, rr, EA, EB);
+      const double xf = dot3(xx, fj);
+      for (int rep = 0; rep < mult; rep++) {
+        s0 = fma(-cm, fma(xf, xx[0] * EA, fj[0] * EB), s0);
+        s1 = fma(-cm, fma(xf, xx[1] * EA, fj[1] * EB), s1);
+        s2 = fma(-cm, fma(xf, xx[2] * EA, fj[2] * EB), s2);
       }
     }
   }
   double dv[3] = {wave_sum(s0), wave_sum(s1), wave_sum(s2)}, dt[3];
   if (fabs(dist) >= fabs(dist1)) {
-    sl_readd_wave(a, cr, blk, m, n, xi, x0, th0, phi0, radPat, c1, c2, dt);
+    readd_wave<true, false>(a, cr, blk, m, n, xi, x0, th0, phi0, radPat, c1, 0., dt);
     for (int d = 0; d < 3; d++) dv[d] += dt[d];
   } else {
     double xi1[3], dv1[3], dv0[3];
-    for (int d = 0; d < 3; d++) xi1[d] = x0[d] + dist1 * a30[d];
-    sl_readd_wave(a, cr, blk, m, n, xi1, x0, th0, phi0, radPat, c1, c2, dv1);
-    sl_readd_wave(a, cr, blk, m, n, x0, x0, th0, phi0, radPat, c1, c2, dv0);
-    if (c2 != 0) {
-      double detJ0, g0[3];
-      spline_interp(blk + vs * SPL_DETJ, m, n, th0, phi0, 1, &detJ0);
-      spline_interp(blk + vs * SPL_G, m, n, th0, phi0, 3, g0);
-      for (int d = 0; d < 3; d++) g0[d] = g0[d] / detJ0;
-      for (int d = 0; d < 3; d++) dv0[d] += (dist > 0 ? 1. : -1.) * c2 * 4 * RBC_PI * g0[d];
-    }
-    for (int d = 0; d < 3; d++) dv[d] += dv0[d] + dist / dist1 * (dv1[d] - dv0[d]);
+    for (int d = 0; d < 3; d++) xi1[d] = fma(dist1, a30[d], x0[d]);
+    readd_wave<true, false>(a, cr, blk, m, n, xi1, x0, th0, phi0, radPat, c1, 0., dv1);
+    readd_wave<true, false>(a, cr, blk, m, n, x0, x0, th0, phi0, radPat, c1, 0., dv0);
+    for (int d = 0; d < 3; d++) dv[d] += fma(dist / dist1, dv1[d] - dv0[d], dv0[d]);
   }
   if (lane == 0)
     for (int d = 0; d < 3; d++) a.dvitem[3 * (size_t)it + d] = dv[d];
@@ -2831,7 +2724,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
   for (int e = apart ? 1 : 0; e < 2; e++) {
     double xe[3];
     for (int d = 0; d < 3; d++) xe[d] = e == 0 ? x0[d] + dist1 * a30[d] : apart ? xi[d] : x0[d];
-    readd_wave<SL>(a, cr, blk, m, n, xe, x0, th0, phi0, radPat, c1, c2, dt);
+    readd_wave<SL, true>(a, cr, blk, m, n, xe, x0, th0, phi0, radPat, c1, c2, dt);
     if (e == 0)
       for (int d = 0; d < 3; d++) dv1[d] = dt[d];
   }
