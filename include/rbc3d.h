@@ -111,6 +111,10 @@ int rbc3d_pair_stats(rbc3d_ctx *ctx, long long *npairs, unsigned long long *chec
  * number of (target, neighbouring cell) projections of RBC_NearSingInt
  * (common/ModRbcSingInt.F90:103-166) and how many passed its distance test. */
 int rbc3d_near_stats(rbc3d_ctx *ctx, long long *nitems, long long *nwork);
+/* Diagnostics of the last add_int_on_rbcs over nT targets: every target's neighbouring
+ * cells (NbrRbcList, common/ModIntOnRbcs.F90), cnt(nT) of them, cell(32,nT) (0-based) and the
+ * closest node's place in the cell's (nlat,nlon) block, node(32,nT) (0-based). */
+int rbc3d_near_lists(rbc3d_ctx *ctx, int nT, int *cnt, int *cell, int *node);
 
 /* --- hot path: PME (common/ModPME.F90) ------------------------------------ */
 /* PME_Distrib_Source(c1,c2,cells,walls) :58-133 (cells/walls = present flags) */

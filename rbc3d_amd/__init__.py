@@ -52,6 +52,7 @@ _SIG = {
     "rbc3d_add_int_on_walls": [C.c_void_p, C.c_double, C.c_int, dp, ip, ip, dp, dp],
     "rbc3d_pair_stats": [C.c_void_p, C.POINTER(C.c_longlong), C.POINTER(C.c_ulonglong)],
     "rbc3d_near_stats": [C.c_void_p, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)],
+    "rbc3d_near_lists": [C.c_void_p, C.c_int, ip, ip, ip],
     "rbc3d_set_geometry_reuse": [C.c_void_p, C.c_int],
     "rbc3d_set_graph": [C.c_void_p, C.c_int],
     "rbc3d_set_deflation": [C.c_void_p, C.c_int],
@@ -516,6 +517,14 @@ class System:
         b = C.c_longlong()
         _call("rbc3d_near_stats", self.h, C.byref(a), C.byref(b))
         return a.value, b.value
+
+    def near_lists(self, nT):
+        """Per target of the last add_int_on_rbcs: {cell: closest node} (0-based; the node's
+        place in the cell's (nlat, nlon) block)."""
+        cnt = np.zeros(nT, np.int32)
+        cell, node = np.zeros((nT, 32), np.int32), np.zeros((nT, 32), np.int32)
+        _call("rbc3d_near_lists", self.h, nT, cnt, cell, node)
+        return [dict(zip(cell[i, :cnt[i]].tolist(), node[i, :cnt[i]].tolist())) for i in range(nT)]
 
     def add_int_on_walls(self, c1, tl, v=None):
         tx, ti, act, A = tl

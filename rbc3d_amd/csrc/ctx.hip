@@ -672,6 +672,7 @@ extern "C" int rbc3d_set_cells(rbc3d_ctx *c, int nrbc, const int *nlat0, const i
     spl += (long long)SPL_NVAR * 2 * g->nlat * g->nlon * 4;
   }
   c->np = np;
+  c->lists_nT = 0;
   c->sbq_ready = false;
   c->x_moved = false;
   c->geom_epoch++;
@@ -873,6 +874,28 @@ extern "C" int rbc3d_near_stats(rbc3d_ctx *c, long long *nitems, long long *nwor
   if (!c) return RBC3D_EINVAL;
   if (nitems) *nitems = c->last_nitems;
   if (nwork) *nwork = c->last_nwork;
+  return RBC3D_OK;
+}
+
+extern "C" int rbc3d_near_lists(rbc3d_ctx *c, int nT, int *cnt, int *cell, int *node) {
+  if (!c || nT < 1 || !cnt || !cell || !node) return RBC3D_EINVAL;
+  if (nT != c->lists_nT) {
+    rbc_set_error("rbc3d_near_lists: no lists of that many targets");
+    return RBC3D_ESTATE;
+  }
+  const size_t n = (size_t)RBC_NBR_MAX * nT;
+  HIP_TRY(hipMemcpyAsync(cnt, c->d_nbr_cnt.p, sizeof(int) * nT, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipMemcpyAsync(cell, c->d_nbr_cell.p, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipMemcpyAsync(node, c->d_nbr_node.p, sizeof(int) * n, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  for (int i = 0; i < nT; i++)
+    for (int k = 0; k < RBC_NBR_MAX; k++) {
+      int &q = node[(size_t)RBC_NBR_MAX * i + k], &cj = cell[(size_t)RBC_NBR_MAX * i + k];
+      if (k < cnt[i])
+        q -= c->cells[cj].off;
+      else
+        q = cj = 0;
+    }
   return RBC3D_OK;
 }
 

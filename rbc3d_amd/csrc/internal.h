@@ -282,6 +282,7 @@ struct rbc3d_ctx {
   bool cell_sol_init = false;
   // last pair statistics
   long long last_npairs = 0, last_nitems = 0, last_nwork = 0;
+  int lists_nT = 0;  // targets whose neighbouring-cell lists are on the device
   // geometry epoch (advanced by set_cells) and the epoch of the geometry-only results
   // kept by the last cacheable add_int_on_rbcs (-1: none)
   int geom_epoch = 0, cache_epoch = -1, cache_nT = 0, cache_nitems = 0, cache_nwork = 0;

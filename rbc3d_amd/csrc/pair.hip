@@ -3098,6 +3098,7 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
   // neighbouring-cell lists
   int *item_off = nullptr, nitems = 0;
   if (!hit) {
+  c->lists_nT = 0;
   RBC_TRY(c->d_nbr_cnt.ensure(2 * (size_t)nT + 2));
   RBC_TRY(c->d_nbr_cell.ensure((size_t)RBC_NBR_MAX * nT + 1));
   RBC_TRY(c->d_nbr_node.ensure((size_t)RBC_NBR_MAX * nT + 1));
@@ -3151,6 +3152,7 @@ int rbc_add_int_on_rbcs_dev(rbc3d_ctx *c, double c1, double c2, int nT, const do
     item_off = c->d_nbr_cnt.p + nT + 1;
     nitems = c->cache_nitems;
   }
+  c->lists_nT = nT;
   c->last_nitems = nitems;
   if (!hit) c->last_nwork = 0;
   // singular and near-singular corrections

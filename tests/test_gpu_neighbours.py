@@ -53,3 +53,56 @@ def test_lists(name):
     print(f"{name}: {count} lists, {g.near_stats()}, matvec {err:.2e}", flush=True)
     assert g.near_stats()[0] == count
     assert err < 1e-12
+
+
+def _edge_points(rng, cells, nl, Lb, rc):
+    """Points whose closest node is nearly a tie (between two nodes next to each other, moved by
+    up to 1e-7 of their distance) or lies at the cut-off's edge, and points anywhere."""
+    L, pts, off = np.asarray(Lb), [], 0
+    for m in nl:
+        x = cells.x[off:off + 6 * m * m].reshape(-1, 3, order="F").reshape(2 * m, m, 3)
+        a3 = cells.a3[off:off + 6 * m * m].reshape(-1, 3, order="F").reshape(2 * m, m, 3)
+        off += 6 * m * m
+        j, i = rng.integers(0, 2 * m, 12), rng.integers(0, m, 12)
+        for other in (x[(j + 1) % (2 * m), i], x[j, (i + 1) % m], x[(j + m) % (2 * m), i]):
+            for e in (0.0, 1e-7, -1e-7, 1e-9):
+                pts.append(x[j, i] * (0.5 + e) + other * (0.5 - e) + rng.choice([0.0, 0.3], (12, 1)) * a3[j, i])
+        for e in (0.0, 1e-7, -1e-7, 1e-13, -1e-13):
+            pts.append(x[j, i] + rc * (1 + e) * a3[j, i])
+    return np.concatenate(pts + [rng.uniform(-0.5, 1.5, (300, 3)) * L])
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_closest_nodes(name):
+    """The lists themselves, cell by cell and node by node, against the oracle's: the cells' own
+    nodes and points at ties and at the cut-off's edge."""
+    import rbc3d_amd as R
+    Lb, rc, n, nlats, lattice = CASES[name]
+    rng = np.random.default_rng(len(name) + 1)
+    if lattice:
+        k = round(n ** (1 / 3))
+        g1 = (np.arange(k) + 0.5) * Lb[0] / k
+        cs = np.stack(np.meshgrid(g1, g1, g1, indexing="ij"), -1).reshape(-1, 3)
+    else:
+        cs = configs.place_centres(rng, n, Lb, 2.1 if n > 3 else 2.0)
+    nl = [nlats[k % len(nlats)] for k in range(n)]
+    cells = configs.build_cells(rng, ["sphere" if lattice else "disc"] * n, nl, [1.0] * n, cs, [1] * n,
+                                rots=[np.eye(3)] * n if lattice else None)
+    w = configs.Workload(name, Lb, configs.alpha_ref_from_xi(2.0), rc, (32,) * 3, 6,
+                         (5.0, 1.0), (0.0, 0.0, 0.0), cells)
+    g, o = R.from_workload(w), O.from_workload(w)
+    x = _edge_points(rng, cells, nl, Lb, rc)
+    k = len(x)
+    free = (x.reshape(-1, order="F").copy(), np.zeros(3 * k, np.int32), np.ones(k, np.int32), np.ones(k))
+    pairs = 0
+    for tl in (free, g.tlist_rbc()):
+        m = len(tl[3])
+        g.add_int_on_rbcs(0.0, 0.0, tl)
+        lists = g.near_lists(m)
+        for i in range(m) if m < 3000 else rng.choice(m, 3000, replace=False):
+            c, cell, il, jl, dist = o.near_list(tl, i)
+            want = {int(a) - 1: (int(b) - 1) + nl[int(a) - 1] * (int(d) - 1) for a, b, d in zip(cell, il, jl)}
+            assert lists[i] == want, (name, i)
+            pairs += c
+    print(f"{name}: {pairs} closest nodes as the oracle's", flush=True)
+    assert pairs > 0
