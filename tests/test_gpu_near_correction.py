@@ -47,3 +47,5 @@ def test_points_near_cells(nlats, c1, c2):
     print(f"grids {nlats}, c {c1}, {c2}: {g.near_stats()}, {err:.2e}, sensitivity {sens:.2e}", flush=True)
     assert g.near_stats()[1] >= k
     assert err < 1e-12 + 16 * sens
+    # the sensitivities measured: up to 4.0e-12 on 6 latitudes' double layer, 7.9e-14 elsewhere
+    assert sens < (1e-11 if c2 != 0 and min(nlats) == 6 else 2e-13)

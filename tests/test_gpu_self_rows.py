@@ -19,6 +19,9 @@ def test_rows(nlats):
     cells = configs.build_cells(rng, ["disc"] * n, nl, [1.0] * n, cs, [1 + k % 2 for k in range(n)])
     w = configs.Workload("rows", (L, L, L), configs.alpha_ref_from_xi(2.0), 2.0, (32,) * 3, 6,
                          (5.0, 1.0), (0.0, 0.0, 0.0), cells)
+    import torch
+    # enough rows for this device to take the path
+    assert 2 * sum(nl) >= torch.cuda.get_device_properties(0).multi_processor_count
     g, o = R.from_workload(w), O.from_workload(w)
     u = rng.standard_normal(g.cell_dof())
     bg, bo = g.cell_matmult(u), o.cell_matmult(u)
