@@ -2513,6 +2513,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   double th0 = r[6], phi0 = r[7], dist = r[11];
   double radPat = cr.radius;
   const double c1 = a.c1;
+  if (c1 == 0) {
+    if (lane < 3) a.dvitem[3 * (size_t)it + lane] = 0.;
+    return;
+  }
   const double *blk = a.spl + cr.spl;
   size_t vs = (size_t)m * n * 4;
   double sizePat = radPat * sqrt(cr.area / (4 * RBC_PI));

@@ -87,3 +87,19 @@ def test_far_targets(L):
         err = np.abs(vg - vo).max() / np.abs(vo).max()
         print(f"box {L}, {c1}, {c2}: {err:.2e}", flush=True)
         assert err < TOL
+
+
+def test_undefined_other_density():
+    """A layer that a sum leaves out does not enter it: the single layer's density undefined, the
+    double layer summed, with and without cells that carry one."""
+    import rbc3d_amd as R
+    for ratios in ((1.0, 1.0), (5.0, 1.0)):
+        w = suspension(13.0, 24, 7, False)
+        w.viscRat = ratios
+        g, o = R.from_workload(w), O.from_workload(w)
+        tl = o.tlist_rbc()
+        vo, _ = o.add_int_on_rbcs(0.0, 0.7, tl)
+        g.set_cell_density(1, np.full_like(w.cells.f, np.nan))
+        vg = g.add_int_on_rbcs(0.0, 0.7, tl)
+        assert g.near_stats()[1] > 0
+        assert np.abs(vg - vo).max() <= TOL * max(np.abs(vo).max(), 1.0), ratios
