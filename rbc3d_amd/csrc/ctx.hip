@@ -636,6 +636,7 @@ extern "C" int rbc3d_set_cells(rbc3d_ctx *c, int nrbc, const int *nlat0, const i
   for (const CellRec &r : c->cells) prev_dof += 3 * r.nlat0 * r.nlat0;
   const int prev_nrbc = c->nrbc;
   c->nrbc = nrbc;
+  c->lists_nT = 0;
   c->cells.resize(nrbc);
   int np = 0, coff = 0;
   long long spl = 0;
@@ -672,7 +673,6 @@ extern "C" int rbc3d_set_cells(rbc3d_ctx *c, int nrbc, const int *nlat0, const i
     spl += (long long)SPL_NVAR * 2 * g->nlat * g->nlon * 4;
   }
   c->np = np;
-  c->lists_nT = 0;
   c->sbq_ready = false;
   c->x_moved = false;
   c->geom_epoch++;
