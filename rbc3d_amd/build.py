@@ -22,8 +22,10 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17",
 # The FP64 constants of the sines, arc cosines and logarithms are hoisted out of the
 # near-singular kernels' loops into some hundred registers by machine-level LICM, which then
 # run at 2 wavefronts a SIMD or spill.  Left in place they are scalar moves beside the vector
-# work: the projection 3.41 -> 3.13 ms, the correction 0.97 -> 0.79 ms (512 cells of 17 x 34
-# nodes); the file's other kernels are unchanged.
+# work.  Without the flag and with it (512 cells of 17 x 34 nodes): correction 1.29 -> 0.80 ms
+# (126 -> 24 spilled registers), projection 3.3 -> 2.96 (214 -> 134 registers); the single
+# layer's pair sums in a tube 0.61 -> 0.59 (12 -> 2 spilled); the file's other kernels lose
+# registers too (k_pair with both layers 154 -> 139, k_nbr 59 -> 54) and change by under 2%.
 FILE_FLAGS = {"pair.hip": ["-mllvm", "-disable-machine-licm"]}
 
 

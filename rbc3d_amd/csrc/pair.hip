@@ -624,15 +624,15 @@ __device__ __forceinline__ void wave_lds_fence() {
 // 64 at a time, one per lane, keeps those within rc of the cluster's bounding sphere, packs
 // their records back to back in its own LDS stage, and evaluates the stage eight sources by
 // eight targets per step; the slots' sums are added by shuffles at the end.  The work is
-// bound by FP64 issue (about 50 instructions a pair) and by the latency of a step's chain
-// (record, distance, table entry), so what matters is how many lanes of a step hold a pair
+// bound by FP64 issue (busy in 72-80% of the cycles; 131 lane instructions a pair in all) and
+// by the latency of a step's chain (record, distance, table entry), so what matters is how many lanes of a step hold a pair
 // within rc and how many wavefronts run: 64 targets sharing a source filled 43% of the
 // lanes of the steps that had any (the chunk is as wide as a fine bin) and paid a step for
 // the candidates that paired with none; eight targets in Z order, which span a third of a
 // bin, fill 56% of all steps.  The sixteen wavefronts of the one workgroup per compute unit
 // share an LDS copy of the double-layer table: a step gathers 64 unrelated entries, which
 // the LDS serves in about 8 cycles per 32 lanes and the vector cache in 64 or more.  Both
-// layers together read their tables from memory and take twelve wavefronts (153 registers).
+// layers together read their tables from memory and take twelve wavefronts (139 registers).
 // Measured, 512 cells at 20% (296k targets, 7.3e8 pairs, double layer): 5.76 ms with 64
 // targets per source, 3.66 so; 128 cells, 20,011 free points, both layers: 1.31 -> 0.75.
 // Two targets a lane (half the record reads, twelve wavefronts): 4.2 ms; the densities read
@@ -1099,11 +1099,12 @@ __global__ void __launch_bounds__(64 * (SL ? 12 : 16)) k_pair(PairArgs a) {
 // fine bin, which its four wavefronts hold in common while they split every 256-source tile
 // between them; the partial sums are added in wavefront order.  Its two tables do not fit
 // the LDS beside the stages of k_pair, and the summation order of a sparse packing feeds a
-// wall solve whose iteration count follows the last bits, so it keeps the order of the
-// sources in the bins.  FILT: the loader drops the sources beyond reach of the chunk's
-// bounding sphere; it pays where bins are dense (a 20% packing: 10% less time) and costs
-// where they are sparse (a tube with ~8 sources per fine bin: 6% more), so the host chooses
-// it by the mean number of sources per fine bin.
+// wall solve whose iteration count follows the last bits, so there (FILT = false) it keeps
+// the order of the sources in the bins.  FILT: the loader drops the sources beyond reach of
+// the chunk's bounding sphere and the wavefronts share out the rest, so a target's order of
+// summation follows its chunk; it pays where bins are dense (a 20% packing: 10% less time)
+// and costs where they are sparse (a tube with ~8 sources per fine bin: 6% more), so the host
+// chooses it by the mean number of sources per fine bin.
 template <bool FILT>
 __global__ void __launch_bounds__(PT *PW) __attribute__((amdgpu_waves_per_eu(6))) k_pair_sl(PairArgs a) {
   __shared__ double sx[PS], sy[PS], sz[PS];
@@ -1888,8 +1889,8 @@ __device__ __forceinline__ void nbr_sweep(const NbrArgs &a, const char *x0, cons
 // within twice the sweep's error bound of its smallest distance (nearly always one) are
 // evaluated in FP64, reduced by (distance, visit key, node).  Cells enter the list in
 // increasing index order.
-// What bounds it: VALU issue (about 11 cells within reach of a target), with the loads of
-// the sweep close behind.  The FP64 sweep behind bounding spheres of 64-node strips that
+// What bounds it: VALU issue, busy in all cycles (about 11 cells within reach of a target),
+// with the loads of the sweep close behind.  The FP64 sweep behind bounding spheres of 64-node strips that
 // was here took some 600 instructions a cell.  296k targets on 512 cells 4.54 -> 1.33
 // ms; on 4096 cells of mixed grids 17.0 -> 5.4 ms; 20,000 points among 128 cells 353 -> 104 us.
 __global__ void __launch_bounds__(NBR_T) k_nbr(NbrArgs a) {
@@ -2401,7 +2402,7 @@ __global__ void k_items(int nT, const int *__restrict__ cnt, const int *__restri
 
 // The single layer's sums of the near-singular correction are written with their
 // contractions: they enter the walls' velocities, whose solver's iteration count hangs on
-// their last bits (traction to 1e-5), so they must not follow what the compiler makes of the
+// their last bits (traction to 3e-5), so they must not follow what the compiler makes of the
 // code around them.  FS: the table's fractions i + 1 - r K and r K - i in one rounding each.
 // (tests/golden/single_layer_near.npz holds the path's values, geometry included.)
 __device__ __forceinline__ double dot3(const double a[3], const double b[3]) {
@@ -2603,9 +2604,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
     for (int d = 0; d < 3; d++) a.dvitem[3 * (size_t)it + d] = dv[d];
 }
 
-// Near-singular stage 2: one wavefront per item that passed the distance test.  Bound by
-// VALU issue (FP64 geometry and splines) and, close behind, by the address unit's rate on the
-// splines' scattered 16-byte loads; the registers limit the wavefronts that hide either.
+// Near-singular stage 2: one wavefront per item that passed the distance test.  VALU issue
+// (FP64 geometry and splines) takes 61-65% of the cycles (49% for both layers at 20,011
+// points); the rest waits, mostly for the splines' scattered 16-byte loads, which the 2.8
+// wavefronts a SIMD that the registers leave do not hide.
 // 512 cells of 17 x 34 nodes 1.17 -> 0.79 ms, 4096 mixed cells 25.5 -> 17.5 ms, by walking
 // only the patch's nodes, the quadrature's roots from a table, and the item's values in
 // scalar registers, which leaves room for 3 wavefronts a SIMD (2: 0.94 ms, 4: 0.86 ms).
