@@ -727,13 +727,14 @@ __global__ void __launch_bounds__(64 * (SL ? 12 : 16)) k_pair(PairArgs a) {
       // The cluster's bounding sphere over its active targets, each taken back into the
       // box (x - kt Lb): a candidate whose image (or minimum image) is farther than
       // rc + r (plus a margin far above the roundings) from the centre is beyond rc of
-      // every target.  All slots hold the same targets.  A cluster with a target thousands
-      // of periods away, whose place in the box has lost digits (or whose bin numbers do not
-      // fit 32 bits), keeps every candidate instead.
+      // every target.  All slots hold the same targets.  A target thousands of periods away,
+      // whose place in the box has lost digits (or whose bin numbers do not fit 32 bits), takes
+      // part with a radius beyond the box instead, so that its cluster keeps every candidate.
       double ct0, ct1, ct2, cut;
       {
-        const double w0 = act ? xi0 - kt0 * L0 : 0., w1 = act ? xi1 - kt1 * L1 : 0.,
-                     w2 = act ? xi2 - kt2 * L2 : 0.;
+        const bool in = act && max(abs(kt0), max(abs(kt1), abs(kt2))) <= 4096;
+        const double w0 = in ? xi0 - kt0 * L0 : 0., w1 = in ? xi1 - kt1 * L1 : 0.,
+                     w2 = in ? xi2 - kt2 * L2 : 0.;
         double s0 = w0, s1 = w1, s2 = w2, n = act ? 1. : 0.;
 #pragma unroll
         for (int o = PC / 2; o > 0; o >>= 1) {
@@ -745,15 +746,13 @@ __global__ void __launch_bounds__(64 * (SL ? 12 : 16)) k_pair(PairArgs a) {
         ct0 = s0 / n;
         ct1 = s1 / n;
         ct2 = s2 / n;
-        double r2 = act ? (w0 - ct0) * (w0 - ct0) + (w1 - ct1) * (w1 - ct1) + (w2 - ct2) * (w2 - ct2)
-                        : 0.;
+        const double far = 4. * (L0 + L1 + L2);
+        double r2 = in    ? (w0 - ct0) * (w0 - ct0) + (w1 - ct1) * (w1 - ct1) + (w2 - ct2) * (w2 - ct2)
+                    : act ? far * far
+                          : 0.;
 #pragma unroll
         for (int o = PC / 2; o > 0; o >>= 1) r2 = fmax(r2, __shfl_xor(r2, o, 64));
         cut = wave_uniform(a.rc * (1. + 1e-9) + sqrt(r2) + 1e-9 * (1. + L0 + L1 + L2));
-        if (__ballot(act && max(abs(kt0), max(abs(kt1), abs(kt2))) > 4096) != 0ull) {
-          ct0 = ct1 = ct2 = 0.;
-          cut = 4. * (L0 + L1 + L2);
-        }
         ct0 = wave_uniform(ct0);
         ct1 = wave_uniform(ct1);
         ct2 = wave_uniform(ct2);
