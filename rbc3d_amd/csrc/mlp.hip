@@ -298,12 +298,12 @@ __device__ __forceinline__ void put_bias(float *red, mlp_f4 v, int lane, bool fi
     for (int i = 0; i < 4; i++) t[i] = o[i] + v[i];
 }
 
-// training: loss and gradient partial sums of one workgroup over the 16-node tiles its
-// MLP_TW wavefronts take in turn; targets are raw increments T[n][3].  A wavefront keeps
+// training: loss and gradient partial sums of one workgroup over the 16-node tiles its first
+// nw <= MLP_TW wavefronts take in turn; targets are raw increments T[n][3].  A wavefront keeps
 // all its sums in registers (160 of them matrix accumulators, one wavefront a SIMD): in
 // LDS, where every tile's products were added before, a tile cost 640 more LDS accesses
 // and 200 lane exchanges for the biases.  65,536 rows: 135 -> 58 us.
-__global__ void __launch_bounds__(MLP_WG, 1) k_mlp_train(int n, const float *__restrict__ X,
+__global__ void __launch_bounds__(MLP_WG, 1) k_mlp_train(int n, int nw, const float *__restrict__ X,
                                                   const float *__restrict__ Tg,
                                                   const unsigned short *__restrict__ wb,
                                                   const float *__restrict__ p,
@@ -329,7 +329,7 @@ __global__ void __launch_bounds__(MLP_WG, 1) k_mlp_train(int n, const float *__r
   #pragma unroll
   for (int t = 0; t < 4; t++) A.w1[t] = A.w4[t] = A.b[0][t] = A.b[1][t] = A.b[2][t] = zero;
   A.b4 = zero;
-  for (int tile = blockIdx.x + gridDim.x * wv; tile < ntile; tile += gridDim.x * MLP_TW) {
+  for (int tile = wv < nw ? blockIdx.x * nw + wv : ntile; tile < ntile; tile += gridDim.x * nw) {
     MlpTile T;
     mlp_forward(sW, sb, X, n, 16 * tile, lane, T);
     const int node = 16 * tile + (lane & 15);
@@ -399,8 +399,8 @@ __global__ void __launch_bounds__(MLP_WG, 1) k_mlp_train(int n, const float *__r
   }
   for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
   if (lane == 0) lred[wv] = lsum;
-  // the wavefronts that had a tile, one after the other: in a small batch the first alone
-  const int nact = min(MLP_TW, (ntile - 1 - (int)blockIdx.x) / (int)gridDim.x + 1);
+  // the wavefronts that had a tile, one after the other
+  const int nact = min(nw, ntile - nw * (int)blockIdx.x);
   for (int w = 0; w < nact; w++) {
     if (w == wv) {
       const bool first = w == 0;
@@ -605,13 +605,13 @@ extern "C" int rbc3d_mlp_forward_dev(rbc3d_mlp *m, int n, const float *d_x, floa
 static int mlp_grad(rbc3d_mlp *m, int n, const float *d_x, const float *d_t, double *loss) {
   hipStream_t st = m->st();
   const int ntile = (n + 15) / 16;
-  // A tile a workgroup up to 256 of them, then more of its wavefronts: the wavefronts add
-  // their sums in turn, some 5 us each (gradient call of 100 rows 67.5 us with four tiles a
-  // workgroup, 53.5 so; 4,096 rows 70 and 62).
-  const int nwg = std::min(256, ntile);
+  // A wavefront a workgroup up to 256 tiles, then more of them: the wavefronts add their sums
+  // in turn, some 5 us each (gradient call of 100 rows 67.5 us with four, 53.5 with one;
+  // 4,096 rows 70 and 62).
+  const int nw = std::min(MLP_TW, (ntile + 255) / 256), nwg = std::min(256, (ntile + nw - 1) / nw);
   RBC_TRY(m->part.ensure((size_t)nwg * GA_N));
   RBC_TRY(m->lpart.ensure(nwg));
-  k_mlp_train<<<nwg, MLP_WG, 0, m->st()>>>(n, d_x, d_t, m->wb.p, m->p.p, m->norm.p,
+  k_mlp_train<<<nwg, MLP_WG, 0, m->st()>>>(n, nw, d_x, d_t, m->wb.p, m->p.p, m->norm.p,
                                                 m->part.p, m->lpart.p);
   k_mlp_reduce<<<(MP_N + 63) / 64, 64 * MLP_RW, 0, m->st()>>>(nwg, m->part.p, m->grad.p);
   HIP_TRY(hipGetLastError());

@@ -10,7 +10,7 @@ from tests.test_gpu_mlp import _data, _net
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 4096, 4097, 16384, 16401])
+@pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 4096, 4097, 8193, 16384, 16401])
 def test_gradient_batches(n):
     import torch
     import rbc3d_amd as R
